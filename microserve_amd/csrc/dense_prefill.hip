@@ -14,7 +14,8 @@
 //    token, q head) pair of the kv head's GQA group, so every K/V operand
 //    read from LDS feeds three MFMAs (244 VGPRs: two waves per SIMD, as the
 //    64 KB of LDS per workgroup allows; three blocks measured 6.7% faster
-//    than two).
+//    than two).  Small grids take one block per wave: three times the
+//    workgroups, each with a shorter chain (kDSmallGrid).
 //  * K/V tiles of 64 keys (256-byte rows) are staged in LDS with direct
 //    global -> LDS loads, double-buffered in separately declared buffers
 //    with one barrier per tile.  Each row's 16-byte chunks are XOR-swizzled
@@ -47,7 +48,6 @@ namespace mskv {
 
 constexpr int kDStep = 64;  // keys per tile
 constexpr int kDWaves = 4;
-constexpr int kDBlocks = 3;  // 16-row blocks per wave
 constexpr int kDThreads = 64 * kDWaves;
 constexpr int kDRow = 2 * kHeadDim;  // bytes per K/V row
 constexpr int kDTile = kDStep * kDRow;
@@ -86,10 +86,12 @@ __device__ __forceinline__ void lds_load16_d(__amdgpu_buffer_rsrc_t r, void* lds
       r, (__attribute__((address_space(3))) void*)lds, 16, (int)off, 0, 0, 0);
 }
 
-template <typename T>
+// kDBlocks: 16-row blocks per wave, 3 or (small grids) 1
+template <typename T, int kDBlocks>
 __global__ __launch_bounds__(kDThreads, 2) void dense_prefill_kernel(DenseArgs a) {
   using A = Act<T>;
   using x8 = typename A::x8;
+  constexpr int kAhead = kDBlocks == 1 ? 4 : 1;
   typedef short i16x4 __attribute__((ext_vector_type(4)));
   __shared__ __attribute__((aligned(16))) uint8_t k_lds0[kDTile];
   __shared__ __attribute__((aligned(16))) uint8_t v_lds0[kDTile];
@@ -199,17 +201,29 @@ __global__ __launch_bounds__(kDThreads, 2) void dense_prefill_kernel(DenseArgs a
     if (t0 >= w_none) return;
     // S^T = K . Q^T: four 16-key tiles, head_dim in four 32-wide chunks
     f32x4 st[kDBlocks][4];
+    // One block per wave: K (and below, V^T) operands are read four MFMAs
+    // ahead, the order pinned; left to the scheduler, most wait for a read
+    // just issued (1000 tokens: 23.8 against 29.8 us).  With three blocks
+    // the other wave covers those waits, and the scheduler's order is 0.6%
+    // faster on 8 x 8192.
+    x8 kring[kAhead];
+    auto read_k = [&](int i) {
+      return __builtin_bit_cast(
+          x8, *reinterpret_cast<const u32x4*>(kt + 16 * (i >> 2) * kDRow + k_off[i & 3]));
+    };
 #pragma unroll
-    for (int tt = 0; tt < 4; ++tt) {
+    for (int i = 0; i < kAhead; ++i) kring[i] = read_k(i);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const x8 ka = __builtin_bit_cast(
-            x8, *reinterpret_cast<const u32x4*>(kt + 16 * tt * kDRow + k_off[c]));
+    for (int i = 0; i < 16; ++i) {
+      const int tt = i >> 2, c = i & 3;
+      if constexpr (kDBlocks == 1) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int b = 0; b < kDBlocks; ++b)
-          st[b][tt] = A::mfma(ka, qop[b][c], c == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : st[b][tt]);
-      }
+      for (int b = 0; b < kDBlocks; ++b)
+        st[b][tt] =
+            A::mfma(kring[i % kAhead], qop[b][c], c == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : st[b][tt]);
+      if (i + kAhead < 16) kring[i % kAhead] = read_k(i + kAhead);
     }
+    if constexpr (kDBlocks == 1) __builtin_amdgcn_sched_barrier(0);
     const bool full = t0 + kDStep <= w_all && t0 + kDStep <= lk;
     if (!full) {
 #pragma unroll
@@ -268,25 +282,32 @@ __global__ __launch_bounds__(kDThreads, 2) void dense_prefill_kernel(DenseArgs a
     // is interleaved with it): 3.7% faster than equal priority, and faster
     // than raising it over the QK^T loop too.
     __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
+    auto read_v = [&](int i) {
+      const int dt = i >> 1, ch = i & 1;
       const uint32_t vo = v_row + ((32u * dt) ^ v_x);
+      const i16x4 r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          reinterpret_cast<__attribute__((address_space(3))) i16x4*>(
+              (__attribute__((address_space(3))) uint8_t*)vt + 32 * ch * kDRow + vo));
+      const i16x4 r1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          reinterpret_cast<__attribute__((address_space(3))) i16x4*>(
+              (__attribute__((address_space(3))) uint8_t*)vt + (32 * ch + 16) * kDRow + vo));
+      typedef short i16x8 __attribute__((ext_vector_type(8)));
+      const i16x8 w = {r0[0], r0[1], r0[2], r0[3], r1[0], r1[1], r1[2], r1[3]};
+      return __builtin_bit_cast(x8, w);
+    };
+    x8 vring[kAhead];
 #pragma unroll
-      for (int ch = 0; ch < 2; ++ch) {
-        const i16x4 r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            reinterpret_cast<__attribute__((address_space(3))) i16x4*>(
-                (__attribute__((address_space(3))) uint8_t*)vt + 32 * ch * kDRow + vo));
-        const i16x4 r1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            reinterpret_cast<__attribute__((address_space(3))) i16x4*>(
-                (__attribute__((address_space(3))) uint8_t*)vt + (32 * ch + 16) * kDRow + vo));
-        const i16x4 lo4 = r0, hi4 = r1;
-        typedef short i16x8 __attribute__((ext_vector_type(8)));
-        const i16x8 w = {lo4[0], lo4[1], lo4[2], lo4[3], hi4[0], hi4[1], hi4[2], hi4[3]};
-        const x8 va = __builtin_bit_cast(x8, w);
+    for (int i = 0; i < kAhead; ++i) vring[i] = read_v(i);
 #pragma unroll
-        for (int b = 0; b < kDBlocks; ++b) acc[b][dt] = A::mfma(va, pv[b][ch], acc[b][dt]);
-      }
+    for (int i = 0; i < 16; ++i) {
+      const int dt = i >> 1, ch = i & 1;
+      if constexpr (kDBlocks == 1) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int b = 0; b < kDBlocks; ++b)
+        acc[b][dt] = A::mfma(vring[i % kAhead], pv[b][ch], acc[b][dt]);
+      if (i + kAhead < 16) vring[i % kAhead] = read_v(i + kAhead);
     }
+    if constexpr (kDBlocks == 1) __builtin_amdgcn_sched_barrier(0);
     // the denominator: sums of the probabilities as rounded for the MFMA,
     // so each output is an exact convex combination of V rows under them
     // (a chain of v_dot2 per pair summed the same rounded values at 4% of
@@ -341,6 +362,43 @@ __global__ __launch_bounds__(kDThreads, 2) void dense_prefill_kernel(DenseArgs a
   }
 }
 
+template <typename T, int kDBlocks>
+static hipError_t launch_dense(const DenseArgs& a, int num_seqs, int max_seqlen_q, hipStream_t st) {
+  const int per_wg = kDWaves * kDBlocks * a.tpr;
+  const dim3 grid((unsigned)(a.hk * a.qgroups), (unsigned)num_seqs,
+                  (unsigned)(((int64_t)max_seqlen_q + per_wg - 1) / per_wg));
+  hipLaunchKernelGGL((dense_prefill_kernel<T, kDBlocks>), grid, dim3(kDThreads), 0, st, a);
+  return hipGetLastError();
+}
+
+// Below this many workgroups of one-block waves, one block per wave.  Two
+// workgroups are resident per CU, 512 on the chip: a grid of about two
+// rounds is bound by its longest workgroup's chain of tiles, and a tile of
+// one block takes 1.1 us against 1.8 us for three.  Larger grids are bound by
+// the matrix and LDS work, where three blocks read each operand a third as
+// often.  Measured, three blocks against one, fp16, causal, 32 q / 8 kv
+// heads unless stated (us; workgroups of the one-block grid):
+//   1000 tokens 35.4 / 23.8 (504), 2000 68.0 / 54.3 (1000), 2500 85.6 / 78.8
+//   (1256), 3000 103.1 / 105.5 (1504); 3 x 1000 43.9 / 45.8 (1512);
+//   64 q heads 1000 39.8 / 30.6 (1000), 2000 80.4 / 90.5 (2000);
+//   40 q heads 2000 71.0 / 63.2 (1336); 16 q heads 4000 117.8 / 83.5 (1000).
+constexpr int64_t kDSmallGrid = 1280;
+
+template <typename T>
+static hipError_t launch_dense_sized(const DenseArgs& a, int num_seqs, int max_seqlen_q,
+                                     hipStream_t st) {
+  // workgroups with rows: no more than the grid holds, and no more than the
+  // tokens fill plus one partial block per sequence
+  const int64_t tok = kDWaves * a.tpr;
+  const int64_t blocks =
+      min((int64_t)num_seqs * ((max_seqlen_q + tok - 1) / tok), a.total_q / tok + num_seqs);
+  // the one-block grid's z must fit its limit too (max_seqlen_q may be far
+  // above the tokens there are)
+  const bool one = blocks * a.hk * a.qgroups <= kDSmallGrid && (max_seqlen_q + tok - 1) / tok <= 65535;
+  return one ? launch_dense<T, 1>(a, num_seqs, max_seqlen_q, st)
+             : launch_dense<T, 3>(a, num_seqs, max_seqlen_q, st);
+}
+
 }  // namespace mskv
 
 extern "C" int mskv_prefill_attention(const void* query, const void* key, const void* value,
@@ -380,17 +438,12 @@ extern "C" int mskv_prefill_attention(const void* query, const void* key, const 
   a.qgroups = (group + 15) / 16;
   a.tpr = 16 / a.gc;
   a.scale_log2 = scale_log2;
-  const int per_wg = mskv::kDWaves * mskv::kDBlocks * a.tpr;
+  const int per_wg = 3 * mskv::kDWaves * a.tpr;
   // grid y and z are limited to 65535
   const int64_t qblocks = ((int64_t)max_seqlen_q + per_wg - 1) / per_wg;
   if (num_seqs > 65535 || qblocks > 65535) return MSKV_EUNSUPPORTED;
-  const dim3 grid((unsigned)(num_kv_heads * a.qgroups), (unsigned)num_seqs,
-                  (unsigned)qblocks);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (act_dtype == MSKV_BFLOAT16)
-    hipLaunchKernelGGL(mskv::dense_prefill_kernel<__bf16>, grid, dim3(mskv::kDThreads), 0, st, a);
-  else
-    hipLaunchKernelGGL(mskv::dense_prefill_kernel<_Float16>, grid, dim3(mskv::kDThreads), 0, st,
-                       a);
-  return (int)hipGetLastError();
+    return (int)mskv::launch_dense_sized<__bf16>(a, num_seqs, max_seqlen_q, st);
+  return (int)mskv::launch_dense_sized<_Float16>(a, num_seqs, max_seqlen_q, st);
 }

@@ -130,3 +130,18 @@ def test_fresh_prefill_random_shapes(case):
     q, k, v, cu_q, cu_k = _setup(8000 + case, lq, lk, hq, hk, dtype)
     if sum(lq):
         _check(q, k, v, cu_q, cu_k, [max(1, x) for x in lq], [max(1, x) for x in lk])
+
+
+@pytest.mark.parametrize("hq,hk,lens", [
+    # one 16-row block per wave: a workgroup covers 16 tokens (group 4),
+    # 12 (group 5), 4 (group 16); tiles of 64 keys
+    (32, 8, [15, 16, 17, 1, 63, 64, 65, 128, 129]), (40, 8, [11, 12, 13, 65]),
+    (16, 1, [3, 4, 5, 64]),
+    # the last length below and the first above the small grid's limit: 1280
+    # workgroups of 16 tokens and 8 heads, and one more
+    (32, 8, [2544]), (32, 8, [2561]),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_fresh_prefill_block_sizes_at_their_edges(hq, hk, lens, dtype):
+    q, k, v, cu_q, cu_k = _setup(451 + sum(lens), lens, lens, hq, hk, dtype)
+    _check(q, k, v, cu_q, cu_k, lens, lens)
