@@ -188,6 +188,38 @@ int mskv_fp8_prefill_attention(const void* query, const void* k_cache,
                                void* stream);
 
 /*
+ * mskv_fp8_prefill_attention with a workspace: where the launch would leave
+ * most of the chip idle (a chunk of a few hundred tokens over a long
+ * prefix), the keys are split over workgroups, whose fp32 partials
+ * ([total_q, num_q_heads, splits, 128] outputs and [total_q, num_q_heads,
+ * splits] log-sum-exps) go to `workspace` and a second kernel merges them.
+ * mskv_fp8_prefill_workspace_bytes gives the bytes it needs, from the
+ * shapes alone: 0 where nothing is split, at most 35 MB.  The workspace
+ * must hold until the work is done and belongs to one call at a time; its
+ * contents on entry do not matter.  A NULL workspace splits nothing; one
+ * that is too small is rejected (MSKV_EWORKSPACE).
+ */
+size_t mskv_fp8_prefill_workspace_bytes(int num_seqs, int64_t total_q,
+                                        int max_seqlen_q, int num_q_heads,
+                                        int num_kv_heads, int head_dim,
+                                        int block_size,
+                                        int max_blocks_per_seq);
+int mskv_fp8_prefill_attention_ws(const void* query, const void* k_cache,
+                                  const void* v_cache,
+                                  const float* k_scale_cache,
+                                  const float* v_scale_cache,
+                                  const int32_t* block_tables,
+                                  const int32_t* cu_seqlens_q,
+                                  const int32_t* cu_seqlens_k, int prefix_len,
+                                  void* out, int num_seqs, int64_t total_q,
+                                  int max_seqlen_q, int num_q_heads,
+                                  int num_kv_heads, int head_dim,
+                                  int block_size, int64_t num_blocks,
+                                  int max_blocks_per_seq, float softmax_scale,
+                                  int act_dtype, void* workspace,
+                                  size_t workspace_bytes, void* stream);
+
+/*
  * Causal varlen attention over unquantized q/k/v: the fresh PREFILL of the
  * FP8-KV path.
  *

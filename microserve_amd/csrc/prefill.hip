@@ -88,7 +88,18 @@ struct PrefillArgs {
   int hq, hk, group, gc, qgroups, tpr, bs, w;
   int gc_magic;  // ceil(256 / gc): n / gc == (n * gc_magic) >> 8 for n < 16
   float scale_log2;
+  // split-KV (small grids): [total_q * hq, splits, 128] outputs and
+  // [total_q * hq, splits] lse values
+  int splits;
+  float* part_o;
+  float* part_lse;
 };
+
+// A key range of at least this many tiles per split
+constexpr int kPMinSplitTiles = 4;
+constexpr int kPMaxSplits = 8;
+// The lse value that marks a row the split kernel has written itself
+constexpr float kPWritten = INFINITY;
 
 __device__ __forceinline__ f32x4 mfma_fp8(const i32x8& a, const i32x8& b, f32x4 c) {
   // compile-time zero scales select the unscaled v_mfma_f32_16x16x128_f8f6f4
@@ -106,7 +117,9 @@ __device__ __forceinline__ void lds_load4(__amdgpu_buffer_rsrc_t r, void* lds, u
       r, (__attribute__((address_space(3))) void*)lds, 4, (int)off, 0, 0, 0);
 }
 
-template <typename T>
+// kSplit: the workgroup takes one of a.splits ranges of the keys (whole
+// tiles, from the actual key count) and leaves partials for the merge.
+template <typename T, bool kSplit>
 __global__ __launch_bounds__(PShape::threads, 2) void prefill_fp8_kernel(PrefillArgs a) {
   using A = Act<T>;
   constexpr int NQ = QuerySplit<T>::parts;
@@ -148,10 +161,40 @@ __global__ __launch_bounds__(PShape::threads, 2) void prefill_fp8_kernel(Prefill
   const int prefix = lk - lq;
   const int wave_tok = kPBlocks * a.tpr;  // query tokens per wave
   const int wg_tok = kPWaves * wave_tok;
-  const int wg_q0 = (int)(gridDim.z - 1 - blockIdx.z) * wg_tok;
+  // grid z: query blocks, of a.splits key ranges each
+  int zb = (int)(gridDim.z - 1 - blockIdx.z), split = 0;
+  if constexpr (kSplit) {
+    split = zb % a.splits;
+    zb /= a.splits;
+  }
+  const int wg_q0 = zb * wg_tok;
   if (wg_q0 >= lq || lq <= 0) return;
   const int wg_qlast = min(lq, wg_q0 + wg_tok) - 1;
-  const int kv_end = min(min(lk, prefix + wg_qlast + 1), a.w * a.bs);
+  int kv_end = min(min(lk, prefix + wg_qlast + 1), a.w * a.bs);
+  int kv_begin = 0;
+  if constexpr (kSplit) {
+    const int tiles = (kv_end + kPStep - 1) / kPStep;
+    const int per = max((tiles + a.splits - 1) / a.splits, kPMinSplitTiles);
+    const bool whole = tiles <= per;  // one range holds all the keys
+    kv_begin = split * per * kPStep;
+    kv_end = min(kv_end, kv_begin + per * kPStep);
+    // a range without keys (unless it is the only one: it writes the rows,
+    // zeros if there are no keys at all) leaves empty partials
+    if (kv_begin >= kv_end && !(whole && split == 0)) {
+      if (whole) return;
+      for (int r = tid; r < kPWaves * kPBlocks * 16; r += PShape::threads) {
+        const int rn = r & 15;
+        const int rq = (rn * a.gc_magic) >> 8;
+        const int qi = wg_q0 + (r >> 4) * a.tpr + rq;
+        const int h = qgi * 16 + rn - rq * a.gc;
+        if (rn < a.tpr * a.gc && qi < lq && h < a.group)
+          a.part_lse[((int64_t)(q_begin + qi) * a.hq + kvh * a.group + h) * a.splits + split] =
+              -INFINITY;
+      }
+      return;
+    }
+    if (whole) split = -1;  // the rows are written here, not merged
+  }
   // keys below w_all are visible to every row of this wave; no row of it
   // sees keys at or above w_none
   const int w_q0 = wg_q0 + wave * wave_tok;
@@ -484,9 +527,9 @@ __global__ __launch_bounds__(PShape::threads, 2) void prefill_fp8_kernel(Prefill
     }
   };
 
-  int valid = stage_tile(0, k_lds0, v_lds0, sc_lds0);
+  int valid = stage_tile(kv_begin, k_lds0, v_lds0, sc_lds0);
   __syncthreads();
-  for (int t0 = 0; t0 < kv_end; t0 += 2 * kPStep) {
+  for (int t0 = kv_begin; t0 < kv_end; t0 += 2 * kPStep) {
     {
       const bool more = t0 + kPStep < kv_end;
       const int valid_next = more ? stage_tile(t0 + kPStep, k_lds1, v_lds1, sc_lds1) : 0;
@@ -509,16 +552,43 @@ __global__ __launch_bounds__(PShape::threads, 2) void prefill_fp8_kernel(Prefill
   // live across the loop, which would spill them.
   int n_out = lane & 15;
   asm volatile("" : "+v"(n_out));
+  // A split workgroup also reads the arguments again: held in scalar
+  // registers across the loop, they spill.
+  int hq = a.hq, group = a.group, gc = a.gc, gc_magic = a.gc_magic, tpr = a.tpr;
+  uint16_t* out = a.out;
+  float *part_o = nullptr, *part_lse = nullptr;
+  int splits = 1;
+  if constexpr (kSplit) {
+    typedef const __attribute__((address_space(4))) PrefillArgs* KernArgs;
+    KernArgs ka = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(ka));
+    hq = ka->hq, group = ka->group, gc = ka->gc, gc_magic = ka->gc_magic, tpr = ka->tpr;
+    out = ka->out;
+    part_o = ka->part_o, part_lse = ka->part_lse, splits = ka->splits;
+  }
 #pragma unroll
   for (int b = 0; b < kPBlocks; ++b) {
     const float lt = lacc[b][0];
-    const int nq = (n_out * a.gc_magic) >> 8;  // n / gc
-    const int qi = w_q0 + b * a.tpr + nq;
-    if (!(n_out < a.tpr * a.gc && qi < lq && qgi * 16 + n_out - nq * a.gc < a.group)) continue;
+    const int nq = (n_out * gc_magic) >> 8;  // n / gc
+    const int qi = w_q0 + b * tpr + nq;
+    if (!(n_out < tpr * gc && qi < lq && qgi * 16 + n_out - nq * gc < group)) continue;
     // acc is in units of fw (a power of two): 1 / fw is exact
     const float scale = lt > 0.0f && fw > 0.0f ? (1.0f / lt) * (1.0f / fw) : 0.0f;
-    const int qhb = kvh * a.group + qgi * 16 + n_out - nq * a.gc;
-    uint16_t* op = a.out + ((int64_t)(q_begin + qi) * a.hq + qhb) * kHeadDim;
+    const int qhb = kvh * group + qgi * 16 + n_out - nq * gc;
+    const int64_t row = (int64_t)(q_begin + qi) * hq + qhb;
+    if constexpr (kSplit) {
+      if (g == 0)
+        part_lse[row * splits + max(split, 0)] =
+            split < 0 ? kPWritten : lt > 0.0f ? m[b] + __log2f(lt) : -INFINITY;
+      if (split >= 0) {
+        float* po = part_o + (row * splits + split) * kHeadDim;
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt)
+          *reinterpret_cast<f32x4*>(po + 16 * dt + 4 * g) = acc[b][dt] * scale;
+        continue;
+      }
+    }
+    uint16_t* op = out + row * kHeadDim;
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) {
       const f32x4 o = acc[b][dt] * scale;
@@ -529,16 +599,134 @@ __global__ __launch_bounds__(PShape::threads, 2) void prefill_fp8_kernel(Prefill
   }
 }
 
+// out[row] = sum_s 2^(lse_s - M) o_s / sum_s 2^(lse_s - M) over the splits
+// that saw keys of the row (zeros if none did).  32 lanes per row, four d
+// each; every split's partial is loaded at once.  HBM-bound: it reads what
+// the split kernel wrote (chunk of 512 over 7680 cached tokens, 4 splits:
+// 34 MB).
+constexpr int kPMergeRows = 8;  // per workgroup
+
+// grid (rows of `tokens` query tokens, sequences): the rows the split
+// kernel's grid covers
+template <typename T, int S>
+__global__ __launch_bounds__(32 * kPMergeRows) void prefill_merge_kernel(
+    const float* __restrict__ part_o, const float* __restrict__ part_lse,
+    const int32_t* __restrict__ cu_q, uint16_t* __restrict__ out, int hq, int64_t total_q,
+    int tokens) {
+  const int local = blockIdx.x * kPMergeRows + (threadIdx.x >> 5);
+  const int i = threadIdx.x & 31;
+  // the sequence's rows, clamped as the split kernel clamps them
+  const int b = blockIdx.y;
+  const int64_t begin = cu_q ? min((int64_t)max(cu_q[b], 0), total_q) : 0;
+  const int64_t end =
+      cu_q ? min(max((int64_t)cu_q[b + 1], begin), total_q) : total_q;
+  if (local >= min((int64_t)tokens, end - begin) * hq) return;
+  const int64_t row = begin * hq + local;
+  float ls[S];
+  f32x4 o[S];
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    ls[s] = part_lse[row * S + s];
+    o[s] = *reinterpret_cast<const f32x4*>(part_o + (row * S + s) * kHeadDim + 4 * i);
+  }
+  if (ls[0] == kPWritten) return;
+  float mm = ls[0];
+#pragma unroll
+  for (int s = 1; s < S; ++s) mm = fmaxf(mm, ls[s]);
+  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+  float den = 0.0f;
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    if (ls[s] != -INFINITY) {  // the partial of an empty range is not written
+      const float w = exp2_fast(ls[s] - mm);
+      den += w;
+      sum += o[s] * w;
+    }
+  }
+  sum *= den > 0.0f ? 1.0f / den : 0.0f;
+  using A = Act<T>;
+  const uint32_t lo = (uint32_t)A::from_f32(sum[0]) | ((uint32_t)A::from_f32(sum[1]) << 16);
+  const uint32_t hi = (uint32_t)A::from_f32(sum[2]) | ((uint32_t)A::from_f32(sum[3]) << 16);
+  *reinterpret_cast<u32x2*>(out + row * kHeadDim + 4 * i) = u32x2{lo, hi};
+}
+
+template <typename T, int S>
+static void launch_merge(const PrefillArgs& a, int num_seqs, int tokens, hipStream_t st) {
+  const int64_t blocks = ((int64_t)tokens * a.hq + kPMergeRows - 1) / kPMergeRows;
+  hipLaunchKernelGGL((prefill_merge_kernel<T, S>), dim3((unsigned)blocks, (unsigned)num_seqs),
+                     dim3(32 * kPMergeRows), 0, st, a.part_o, a.part_lse, a.cu_q, a.out, a.hq,
+                     a.total_q, tokens);
+}
+
+template <typename T>
+static hipError_t launch_prefill(const PrefillArgs& a, int num_seqs, int64_t qblocks,
+                                 hipStream_t st) {
+  dim3 grid((unsigned)(a.hk * a.qgroups), (unsigned)num_seqs, (unsigned)qblocks);
+  if (a.splits <= 1) {
+    hipLaunchKernelGGL((prefill_fp8_kernel<T, false>), grid, dim3(PShape::threads), 0, st, a);
+    return hipGetLastError();
+  }
+  grid.z *= (unsigned)a.splits;
+  hipLaunchKernelGGL((prefill_fp8_kernel<T, true>), grid, dim3(PShape::threads), 0, st, a);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  // the tokens of a sequence that the grid covers
+  const int tokens = (int)min(qblocks * 8 * a.tpr, a.total_q);
+  switch (a.splits) {
+    case 2: launch_merge<T, 2>(a, num_seqs, tokens, st); break;
+    case 3: launch_merge<T, 3>(a, num_seqs, tokens, st); break;
+    case 4: launch_merge<T, 4>(a, num_seqs, tokens, st); break;
+    case 5: launch_merge<T, 5>(a, num_seqs, tokens, st); break;
+    case 6: launch_merge<T, 6>(a, num_seqs, tokens, st); break;
+    case 7: launch_merge<T, 7>(a, num_seqs, tokens, st); break;
+    default: launch_merge<T, 8>(a, num_seqs, tokens, st); break;
+  }
+  return hipGetLastError();
+}
+
+// Key ranges per workgroup, from shapes alone.  Two workgroups are resident
+// per CU, 512 on the chip, and a second one costs the first little (a tile
+// takes 3.2 us alone, 3.9 us beside another), so a grid of at most 256 is
+// split until it fills them; the merge reads and writes 1 KB per row and
+// split, so a range keeps at least kPMinSplitTiles tiles.
+static int prefill_splits(int num_seqs, int64_t max_seqlen_q, int num_q_heads, int num_kv_heads,
+                          int block_size, int max_blocks_per_seq) {
+  const int group = num_q_heads / num_kv_heads;
+  const int per_wg = 8 * (group < 16 ? 16 / group : 1);
+  const int64_t qblocks = (max_seqlen_q + per_wg - 1) / per_wg;
+  const int64_t wgs = num_seqs * qblocks * num_kv_heads * ((group + 15) / 16);
+  if (wgs <= 0) return 1;
+  const int64_t tiles = (int64_t)max_blocks_per_seq * block_size / kPStep;
+  const int64_t s = min(min((int64_t)512 / wgs, tiles / kPMinSplitTiles), (int64_t)kPMaxSplits);
+  // (256 workgroups of 128 rows: far from any limit of the grids)
+  if (s < 2) return 1;
+  return (int)s;
+}
+
 }  // namespace mskv
 
-extern "C" int mskv_fp8_prefill_attention(
+extern "C" size_t mskv_fp8_prefill_workspace_bytes(int num_seqs, int64_t total_q, int max_seqlen_q,
+                                                   int num_q_heads, int num_kv_heads,
+                                                   int head_dim, int block_size,
+                                                   int max_blocks_per_seq) {
+  if (num_seqs <= 0 || total_q <= 0 || max_seqlen_q <= 0 || num_q_heads <= 0 ||
+      num_kv_heads <= 0 || num_q_heads % num_kv_heads != 0 || head_dim != mskv::kHeadDim ||
+      block_size <= 0 || block_size % mskv::kPStep != 0 || max_blocks_per_seq <= 0)
+    return 0;
+  const int s = mskv::prefill_splits(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads,
+                                     block_size, max_blocks_per_seq);
+  return s < 2 ? 0 : (size_t)total_q * num_q_heads * s * (mskv::kHeadDim + 1) * sizeof(float);
+}
+
+extern "C" int mskv_fp8_prefill_attention_ws(
     const void* query, const void* k_cache, const void* v_cache,
     const float* k_scale_cache, const float* v_scale_cache,
     const int32_t* block_tables, const int32_t* cu_seqlens_q,
     const int32_t* cu_seqlens_k, int prefix_len, void* out, int num_seqs,
     int64_t total_q, int max_seqlen_q, int num_q_heads, int num_kv_heads,
     int head_dim, int block_size, int64_t num_blocks, int max_blocks_per_seq,
-    float softmax_scale, int act_dtype, void* stream) {
+    float softmax_scale, int act_dtype, void* workspace, size_t workspace_bytes,
+    void* stream) {
   if (num_seqs < 0 || total_q < 0 || max_seqlen_q < 0 || num_q_heads <= 0 ||
       num_kv_heads <= 0 || block_size <= 0 || num_blocks < 0 ||
       max_blocks_per_seq <= 0 || prefix_len < 0)
@@ -586,14 +774,38 @@ extern "C" int mskv_fp8_prefill_attention(
   // grid y and z are limited to 65535
   const int64_t qblocks = ((int64_t)max_seqlen_q + per_wg - 1) / per_wg;
   if (num_seqs > 65535 || qblocks > 65535) return MSKV_EUNSUPPORTED;
-  const dim3 grid((unsigned)(num_kv_heads * a.qgroups), (unsigned)num_seqs,
-                  (unsigned)qblocks);
+  // without a workspace, one workgroup walks all the keys of its rows
+  a.splits = 1;
+  a.part_o = a.part_lse = nullptr;
+  if (workspace) {
+    const size_t need = mskv_fp8_prefill_workspace_bytes(num_seqs, total_q, max_seqlen_q,
+                                                         num_q_heads, num_kv_heads, head_dim,
+                                                         block_size, max_blocks_per_seq);
+    if (workspace_bytes < need) return MSKV_EWORKSPACE;
+    if (need > 0) {
+      a.splits = mskv::prefill_splits(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads,
+                                      block_size, max_blocks_per_seq);
+      a.part_o = (float*)workspace;
+      a.part_lse = a.part_o + (size_t)total_q * num_q_heads * a.splits * head_dim;
+    }
+  }
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (act_dtype == MSKV_BFLOAT16)
-    hipLaunchKernelGGL(mskv::prefill_fp8_kernel<__bf16>, grid,
-                       dim3(mskv::PShape::threads), 0, s, a);
-  else
-    hipLaunchKernelGGL(mskv::prefill_fp8_kernel<_Float16>, grid,
-                       dim3(mskv::PShape::threads), 0, s, a);
-  return (int)hipGetLastError();
+    return (int)mskv::launch_prefill<__bf16>(a, num_seqs, qblocks, s);
+  return (int)mskv::launch_prefill<_Float16>(a, num_seqs, qblocks, s);
+}
+
+extern "C" int mskv_fp8_prefill_attention(
+    const void* query, const void* k_cache, const void* v_cache,
+    const float* k_scale_cache, const float* v_scale_cache,
+    const int32_t* block_tables, const int32_t* cu_seqlens_q,
+    const int32_t* cu_seqlens_k, int prefix_len, void* out, int num_seqs,
+    int64_t total_q, int max_seqlen_q, int num_q_heads, int num_kv_heads,
+    int head_dim, int block_size, int64_t num_blocks, int max_blocks_per_seq,
+    float softmax_scale, int act_dtype, void* stream) {
+  return mskv_fp8_prefill_attention_ws(
+      query, k_cache, v_cache, k_scale_cache, v_scale_cache, block_tables, cu_seqlens_q,
+      cu_seqlens_k, prefix_len, out, num_seqs, total_q, max_seqlen_q, num_q_heads, num_kv_heads,
+      head_dim, block_size, num_blocks, max_blocks_per_seq, softmax_scale, act_dtype, nullptr, 0,
+      stream);
 }

@@ -23,6 +23,30 @@ def _check_common(query, k_cache, v_cache, k_scale_cache, v_scale_cache):
                    v_scale_cache)
 
 
+def _launch(lib, what, query, caches, tables, cu_q, cu_k, prefix_len, output, num_seqs,
+            max_seqlen_q, max_blocks, softmax_scale):
+    """One prefill launch.  The split partials' workspace, where the shapes
+    need one, is allocated per call on the current stream, which the kernels
+    run on: the caching allocator reuses it in stream order, and a graph
+    capture takes it from its own pool."""
+    k_cache, v_cache, k_scale_cache, v_scale_cache = caches
+    total_q, num_q_heads, head_dim = query.shape
+    num_blocks, block_size, num_kv_heads = k_cache.shape[:3]
+    ws_bytes = lib.mskv_fp8_prefill_workspace_bytes(
+        num_seqs, total_q, max_seqlen_q, num_q_heads, num_kv_heads, head_dim, block_size,
+        max_blocks)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=query.device) if ws_bytes else None
+    status = lib.mskv_fp8_prefill_attention_ws(
+        query.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+        k_scale_cache.data_ptr(), v_scale_cache.data_ptr(), tables.data_ptr(),
+        None if cu_q is None else cu_q.data_ptr(), None if cu_k is None else cu_k.data_ptr(),
+        prefix_len, output.data_ptr(), num_seqs, total_q, max_seqlen_q, num_q_heads,
+        num_kv_heads, head_dim, block_size, num_blocks, max_blocks, float(softmax_scale),
+        _lib.act_dtype(query), None if ws is None else ws.data_ptr(), ws_bytes,
+        _lib.stream_of(query))
+    _lib.check(status, what)
+
+
 def fp8_chunk_prefill_attention(
     query: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     k_scale_cache: torch.Tensor, v_scale_cache: torch.Tensor,
@@ -44,7 +68,7 @@ def fp8_chunk_prefill_attention(
     del block_m, block_n
     query = query.contiguous()
     block_table = block_table.contiguous().view(-1)
-    query_len, num_q_heads, head_dim = query.shape
+    query_len = query.shape[0]
     _check_common(query, k_cache, v_cache, k_scale_cache, v_scale_cache)
     assert block_table.dtype == torch.int32
     _lib.on_device("fp8_chunk_prefill_attention", query, block_table)
@@ -53,15 +77,9 @@ def fp8_chunk_prefill_attention(
     output = torch.empty_like(query)
     if query_len == 0:
         return output
-    lib = _lib.load()
-    status = lib.mskv_fp8_prefill_attention(
-        query.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-        k_scale_cache.data_ptr(), v_scale_cache.data_ptr(),
-        block_table.data_ptr(), None, None, prefix_len, output.data_ptr(),
-        1, query_len, query_len, num_q_heads, k_cache.shape[2], head_dim,
-        k_cache.shape[1], k_cache.shape[0], block_table.numel(),
-        float(softmax_scale), _lib.act_dtype(query), _lib.stream_of(query))
-    _lib.check(status, "fp8_chunk_prefill_attention")
+    _launch(_lib.load(), "fp8_chunk_prefill_attention", query,
+            (k_cache, v_cache, k_scale_cache, v_scale_cache), block_table, None, None, prefix_len,
+            output, 1, query_len, block_table.numel(), softmax_scale)
     return output
 
 
@@ -85,7 +103,7 @@ def fp8_varlen_prefill_attention(
     block_tables = block_tables.contiguous()
     cu_seqlens_q = cu_seqlens_q.contiguous()
     cu_seqlens_k = cu_seqlens_k.contiguous()
-    total_q, num_q_heads, head_dim = query.shape
+    total_q = query.shape[0]
     _check_common(query, k_cache, v_cache, k_scale_cache, v_scale_cache)
     assert block_tables.dtype == cu_seqlens_q.dtype == cu_seqlens_k.dtype == torch.int32
     num_seqs = cu_seqlens_q.numel() - 1
@@ -96,14 +114,8 @@ def fp8_varlen_prefill_attention(
     output = torch.empty_like(query)
     if total_q == 0 or num_seqs == 0:
         return output
-    lib = _lib.load()
-    status = lib.mskv_fp8_prefill_attention(
-        query.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-        k_scale_cache.data_ptr(), v_scale_cache.data_ptr(),
-        block_tables.data_ptr(), cu_seqlens_q.data_ptr(),
-        cu_seqlens_k.data_ptr(), 0, output.data_ptr(), num_seqs, total_q,
-        int(max_seqlen_q), num_q_heads, k_cache.shape[2], head_dim,
-        k_cache.shape[1], k_cache.shape[0], block_tables.shape[1],
-        float(softmax_scale), _lib.act_dtype(query), _lib.stream_of(query))
-    _lib.check(status, "fp8_varlen_prefill_attention")
+    _launch(_lib.load(), "fp8_varlen_prefill_attention", query,
+            (k_cache, v_cache, k_scale_cache, v_scale_cache), block_tables, cu_seqlens_q,
+            cu_seqlens_k, 0, output, num_seqs, int(max_seqlen_q), block_tables.shape[1],
+            softmax_scale)
     return output

@@ -262,3 +262,44 @@ def test_chunk_prefill_single_equals_varlen():
     b = fp8_varlen_prefill_attention(query.to(H.DEV), *caches, tables.to(H.DEV),
                                      cu_q.to(H.DEV), cu_k.to(H.DEV), 100, 0.088)
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hk,lq,lk,width", [
+    # 32 tokens per workgroup (group 4), 128-key tiles, four tiles at least
+    # per range: the last key of a range, the first of the next, one tile less
+    (32, 8, [31], [31 + 1024 - 31], 0), (32, 8, [32], [1025], 0), (32, 8, [33], [1024 + 129], 0),
+    # the most ranges (8), keys that end inside the last
+    (16, 8, [17], [17 + 5000], 0),
+    # a table far wider than the keys: most ranges are empty, or one holds all
+    (32, 8, [40], [40 + 600], 64), (32, 8, [40], [40 + 300], 64),
+    # sequences of different key counts (one range, several), none, one token
+    (32, 8, [20, 0, 64, 1], [20 + 100, 700, 64 + 3000, 1 + 2100], 0),
+    # lanes past the group's heads (5 of 16 rows idle per block), group above 16
+    (40, 8, [50], [50 + 2000], 0), (24, 1, [30], [30 + 2500], 0),
+])
+def test_prefill_split_ranges_at_their_edges(hq, hk, lq, lk, width, dtype):
+    """Grids that leave the chip idle split the keys over workgroups; the
+    merged result must match the oracle wherever the ranges end."""
+    query, tables, caches, cu_q, cu_k = _varlen_setup(281 + sum(lq), lq, lk, hq, hk, dtype)
+    if width:
+        tables = torch.nn.functional.pad(tables, (0, width - tables.shape[1]), value=-1)
+    _varlen_check(query, tables, caches, cu_q, cu_k, lq)
+
+
+def test_prefill_split_under_capture_replays_the_eager_result():
+    """The split partials' workspace is allocated per call, under capture
+    from the graph's pool; replays between eager calls give the same bits."""
+    query, tables, caches, cu_q, cu_k = _varlen_setup(291, [64], [64 + 3000], 32, 8)
+    q, t = query.to(H.DEV), tables.to(H.DEV)
+    eager = fp8_chunk_prefill_attention(q, *caches, t, 3000, 0.088)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = fp8_chunk_prefill_attention(q, *caches, t, 3000, 0.088)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        again = fp8_chunk_prefill_attention(q, *caches, t, 3000, 0.088)
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager) and torch.equal(again, eager)
