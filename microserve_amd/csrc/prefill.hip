@@ -96,7 +96,7 @@ struct PrefillArgs {
 };
 
 // A key range of at least this many tiles per split
-constexpr int kPMinSplitTiles = 4;
+constexpr int kPMinSplitTiles = 2;
 constexpr int kPMaxSplits = 8;
 // The lse value that marks a row the split kernel has written itself
 constexpr float kPWritten = INFINITY;
@@ -687,8 +687,12 @@ static hipError_t launch_prefill(const PrefillArgs& a, int num_seqs, int64_t qbl
 // Key ranges per workgroup, from shapes alone.  Two workgroups are resident
 // per CU, 512 on the chip, and a second one costs the first little (a tile
 // takes 3.2 us alone, 3.9 us beside another), so a grid of at most 256 is
-// split until it fills them; the merge reads and writes 1 KB per row and
-// split, so a range keeps at least kPMinSplitTiles tiles.
+// split until it fills them (768 or 1024 instead: 120-134 against 106 us on
+// 512 new over 7680 cached tokens); a range
+// keeps kPMinSplitTiles tiles, below which the merge's 1 KB per row and
+// split costs what the shorter chain saves.  Unsplit against split (fp16,
+// 32 q / 8 kv heads, new/cached, with the store, us): 512/7680 210 -> 106,
+// 128/7680 195 -> 53, 64/2000 66 -> 31, 512/1000 54 -> 46, 256/600 39 -> 35.
 static int prefill_splits(int num_seqs, int64_t max_seqlen_q, int num_q_heads, int num_kv_heads,
                           int block_size, int max_blocks_per_seq) {
   const int group = num_q_heads / num_kv_heads;

@@ -266,7 +266,7 @@ def test_chunk_prefill_single_equals_varlen():
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("hq,hk,lq,lk,width", [
-    # 32 tokens per workgroup (group 4), 128-key tiles, four tiles at least
+    # 32 tokens per workgroup (group 4), 128-key tiles, two tiles at least
     # per range: the last key of a range, the first of the next, one tile less
     (32, 8, [31], [31 + 1024 - 31], 0), (32, 8, [32], [1025], 0), (32, 8, [33], [1024 + 129], 0),
     # the most ranges (8), keys that end inside the last
