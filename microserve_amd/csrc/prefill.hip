@@ -688,11 +688,12 @@ static hipError_t launch_prefill(const PrefillArgs& a, int num_seqs, int64_t qbl
 // per CU, 512 on the chip, and a second one costs the first little (a tile
 // takes 3.2 us alone, 3.9 us beside another), so a grid of at most 256 is
 // split until it fills them (768 or 1024 instead: 120-134 against 106 us on
-// 512 new over 7680 cached tokens); a range
-// keeps kPMinSplitTiles tiles, below which the merge's 1 KB per row and
-// split costs what the shorter chain saves.  Unsplit against split (fp16,
-// 32 q / 8 kv heads, new/cached, with the store, us): 512/7680 210 -> 106,
-// 128/7680 195 -> 53, 64/2000 66 -> 31, 512/1000 54 -> 46, 256/600 39 -> 35.
+// 512 new over 7680 cached tokens), where the shorter chain saves more than
+// the merge costs: its launch, 5 us, and 1 KB per row and split at 6 TB/s.
+// Unsplit against split (fp16, 32 q / 8 kv heads, new/cached, with the
+// store, us): 512/7680 210 -> 106, 128/7680 195 -> 53, 64/2000 66 -> 31,
+// 512/1000 54 -> 46, 256/600 39 -> 35; split all the same, 4 x 74/129 went
+// 12.5 -> 18.0 and 509/200 at 64 q heads 33.8 -> 35.8.
 static int prefill_splits(int num_seqs, int64_t max_seqlen_q, int num_q_heads, int num_kv_heads,
                           int block_size, int max_blocks_per_seq) {
   const int group = num_q_heads / num_kv_heads;
@@ -701,10 +702,19 @@ static int prefill_splits(int num_seqs, int64_t max_seqlen_q, int num_q_heads, i
   const int64_t wgs = num_seqs * qblocks * num_kv_heads * ((group + 15) / 16);
   if (wgs <= 0) return 1;
   const int64_t tiles = (int64_t)max_blocks_per_seq * block_size / kPStep;
-  const int64_t s = min(min((int64_t)512 / wgs, tiles / kPMinSplitTiles), (int64_t)kPMaxSplits);
-  // (256 workgroups of 128 rows: far from any limit of the grids)
-  if (s < 2) return 1;
-  return (int)s;
+  const int64_t most =
+      min(min((int64_t)512 / wgs, tiles / kPMinSplitTiles), (int64_t)kPMaxSplits);
+  const double rows = (double)wgs * 8 * 16;
+  int best = 1;
+  double best_saved = 2.0;  // us: the table bounds the keys from above only
+  for (int s = 2; s <= most; ++s) {
+    const double saved = 3.2 * (double)(tiles - (tiles + s - 1) / s) - 5.0 - rows * s * 1.7e-4;
+    if (saved > best_saved) {
+      best = s;
+      best_saved = saved;
+    }
+  }
+  return best;
 }
 
 }  // namespace mskv
