@@ -38,8 +38,9 @@
 //    only when a head's max grows by more than 2^8.
 //  * Tiles are double-buffered in LDS: step i+1's rows are staged while
 //    step i is consumed, so the K/V registers live only while in flight.
-//  * Split-KV: the host picks pages-per-split from shapes only; each split
-//    writes (o / l, m + log2 l) partials and a second kernel merges them:
+//  * Split-KV: the host picks the split count from shapes only; small grids
+//    choose the tokens per split on the device, from the lengths
+//    (split_tokens_of); each split writes (o / l, m + log2 l) partials and a second kernel merges them:
 //    decode_combine_small_kernel up to 8 splits, decode_combine_kernel up
 //    to 64, decode_combine_wide_kernel beyond (an in-kernel merge needs
 //    agent-scope fences, i.e. an L2 writeback + invalidate per XCD, which
@@ -59,6 +60,7 @@
 //    tokens are masked, so a bad table entry cannot fault.
 #include <math.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "mskv_device.h"
@@ -71,12 +73,15 @@ constexpr int kStep = 32;  // tokens per inner step (one LDS K/V tile pair)
 // p < 2^8 every weight stays below 2^15, inside fp16's range
 constexpr float kPvScaleMax = 128.0f;
 constexpr int kMaxPagesPerSplit = 4;
+constexpr int kMinSplitSteps = 2;  // steps of a split whose size follows the lengths
 // Split-KV aims at this many waves: eight per CU
 constexpr int kTargetWaves = 2048;
 // Waves of one workgroup take consecutive kv heads of the same tokens, so a
 // workgroup streams whole contiguous token rows; the waves never synchronize
 // with each other.
 constexpr int kWavesPerWG = 8;
+// Largest split partials that splits finer than a page may ask for
+constexpr int64_t kFinePartialBytes = 16 << 20;
 constexpr int kNarrowWaves = 4;       // workgroup shape for grids of many rounds
 constexpr int64_t kWideGridMax = 512; // 8-wave workgroups: about two rounds
 // Largest split-partials scratch the allocation-free entry point serves
@@ -89,6 +94,18 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
+
+// How the splits of a launch are laid out: split i of a sequence holds its
+// tokens [i * split_tokens, (i + 1) * split_tokens).
+struct SplitRule {
+  int batch, splits;
+  int fixed;       // split_tokens from the shapes: a whole number of pages
+  int max_tokens;  // addressable tokens of a sequence (the table's width)
+  bool adapt;      // split_tokens follows the lengths, else it is `fixed`
+  // 1 / the splits that run at once (CUs over workgroups per split, less
+  // half a split per sequence), and 1 / splits
+  float inv_slots, inv_splits;
+};
 
 struct DecodeArgs {
   const uint16_t* q;
@@ -108,9 +125,82 @@ struct DecodeArgs {
   const int4* items;
   const int* item_count;
   int batch, hq, hk, group, qgroups, bs, w, splits, pages_per_split;
+  SplitRule rule;
   int64_t num_blocks;
   float scale_log2;
 };
+
+// Sum / max over the wave with DPP row shifts and the two cross-row swaps
+// (no LDS round trip).
+__device__ __forceinline__ int wave_sum_i32(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);   // quad_perm [1,0,3,2]
+  v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false);   // quad_perm [2,3,0,1]
+  v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, false);  // row_half_mirror
+  v += __builtin_amdgcn_update_dpp(0, v, 0x140, 0xF, 0xF, false);  // row_mirror
+  const auto r16 = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
+  v = (int)(r16[0] + r16[1]);
+  const auto r32 = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
+  return (int)(r32[0] + r32[1]);
+}
+__device__ __forceinline__ int wave_max_u31(int v) {  // of values >= 0
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x140, 0xF, 0xF, false));
+  const auto r16 = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
+  v = max((int)r16[0], (int)r16[1]);
+  const auto r32 = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
+  return max((int)r32[0], (int)r32[1]);
+}
+
+// The tokens per split of this step, from the lengths on the device: a
+// table as wide as the longest context a graph was captured for says
+// nothing about the lengths, and a wave's chain of 32-token steps (about 2
+// us each) sets the time of a small step.  The splits of all sequences
+// should run at once, so the tokens spread over the slots (less half a
+// split per sequence for its ragged end); a split has two steps at least,
+// the longest sequence fits in the splits there are, and the shape's own
+// split, which fills the chip when every sequence is full, is the most.
+// Whole steps, not whole pages.  Measured against the shape's split, us:
+// batch 16, 64 to 4096 tokens under 128-entry tables 77 -> 23 (the layer's
+// step), 8 x 1000 under 128 entries 53 -> 13, 1 x 512 18.6 -> 11.2, 1 x 4096
+// 19.4 -> 13.2.  Every wave of the split kernel and of the
+// merges computes the same value.  (batch <= 256 and max_tokens <= 2^22
+// where it adapts: the sum of steps stays within an int.)
+// `own` is this lane's length, loaded early so that it shares the round trip
+// of the caller's first reads; `len` is the caller's sequence's.
+__device__ __forceinline__ int lane_length(const int32_t* __restrict__ seqlens,
+                                           const SplitRule& r) {
+  const int lane = threadIdx.x & 63;
+  return r.adapt && r.batch > 1 && lane < r.batch ? seqlens[lane] : 0;
+}
+__device__ __forceinline__ int split_tokens_of(int own, int len,
+                                               const int32_t* __restrict__ seqlens,
+                                               const SplitRule& r) {
+  if (!r.adapt) return r.fixed;
+  int steps, longest;
+  auto steps_of = [&](int len) {
+    return (max(0, min(len, r.max_tokens)) + kStep - 1) / kStep;
+  };
+  if (r.batch == 1) {
+    steps = longest = steps_of(len);
+  } else {
+    steps = longest = steps_of(own);
+    for (int i = 64 + (threadIdx.x & 63); i < r.batch; i += 64) {
+      const int n = steps_of(seqlens[i]);
+      steps += n;
+      longest = max(longest, n);
+    }
+    steps = __builtin_amdgcn_readfirstlane(wave_sum_i32(steps));
+    longest = __builtin_amdgcn_readfirstlane(wave_max_u31(longest));
+  }
+  // (longest / splits is at least 1 / longest away from a whole number or on
+  // it, 2^-17 with these limits, so the float product never rounds it down
+  // past one)
+  const int per = max((int)ceilf(fmaxf((float)steps * r.inv_slots, (float)longest * r.inv_splits)),
+                      kMinSplitSteps);
+  return min(per * kStep, r.fixed);
+}
 
 struct StepLoads {
   u32x4 k[4], v[4];      // K/V rows 8c + lane/8, 16-byte chunk lane%8
@@ -386,11 +476,17 @@ void decode_fp8_kernel(DecodeArgs a) {
   // together, first thing, so the first K/V loads wait for one memory round
   // trip, not a chain of them (readfirstlane is convergent, so the compiler
   // cannot sink a read below the branches that use it).  The split's first
-  // page is inside the table: split * pages_per_split < w for every split
-  // count the host accepts.  With work items, grid row (z, y) takes item
-  // z * splits + y: the valid splits of the longest sequences first, short
-  // sequences' in the last round, and the rows past the last item (empty
-  // splits) at the end of the grid.
+  // page, clamped to the table (splits finer than a page may be more than its
+  // entries), is that of the shape's own split; another one is read below.
+  // With work items, grid row (z, y) takes item z * splits + y: the valid
+  // splits of the longest sequences first, short sequences' in the last
+  // round, and the rows past the last item (empty splits) at the end of the
+  // grid.  Splits that follow the lengths put the empty ones last by taking
+  // z as the split (in between, every 2 us wave of them delays the valid ones
+  // behind: batch 16 x 4096 tokens, half of 32 splits empty, 43 against 29
+  // us); the sequences rotate with it, so that one sequence's splits spread
+  // over the XCDs.
+  const int own = lane_length(a.seqlens, a.rule);
   int b, split, len_raw, blk_first;
   if (a.items) {
     const int item = blockIdx.z * a.splits + blockIdx.y;
@@ -403,18 +499,18 @@ void decode_fp8_kernel(DecodeArgs a) {
     if (item >= count) return;
     if ((unsigned)b >= (unsigned)a.batch || (unsigned)split >= (unsigned)a.splits) return;
   } else {
-    split = blockIdx.y;
-    b = blockIdx.z;
+    split = a.rule.adapt ? blockIdx.z : blockIdx.y;
+    b = a.rule.adapt ? (blockIdx.y + blockIdx.z) % a.batch : blockIdx.z;
     len_raw = __builtin_amdgcn_readfirstlane(a.seqlens[b]);
-    blk_first =
-        __builtin_amdgcn_readfirstlane(a.bt[(int64_t)b * a.w + split * a.pages_per_split]);
+    blk_first = __builtin_amdgcn_readfirstlane(
+        a.bt[(int64_t)b * a.w + min(split * a.pages_per_split, a.w - 1)]);
   }
   if (unit >= a.hk * a.qgroups) return;
   const int kvh = unit / a.qgroups;
   const int hig = (unit - kvh * a.qgroups) * 16 + n;  // head within its group
   const bool head_ok = hig < a.group;
   const int qh = kvh * a.group + hig;
-  const int split_tokens = a.pages_per_split * a.bs;
+  const int split_tokens = a.items ? a.rule.fixed : split_tokens_of(own, len_raw, a.seqlens, a.rule);
   const int t_begin = split * split_tokens;
   // tokens past the block table's width are not addressable: ignore them
   const int L = min(len_raw, a.w * a.bs);
@@ -430,6 +526,8 @@ void decode_fp8_kernel(DecodeArgs a) {
   }
   if (t_begin >= L) return;
   const int t_end = min(L, t_begin + split_tokens);
+  if (split_tokens != a.rule.fixed)
+    blk_first = __builtin_amdgcn_readfirstlane(a.bt[(int64_t)b * a.w + t_begin / a.bs]);
 
   f32x4 acc[8];
   float m, l;
@@ -584,12 +682,15 @@ template <typename T>
 __global__ __launch_bounds__(64) void decode_combine_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_lse,
     const int32_t* __restrict__ seqlens, uint16_t* __restrict__ out, int hq,
-    int splits, int split_tokens, int max_tokens) {
+    SplitRule rule) {
+  const int splits = rule.splits;
+  const int own = lane_length(seqlens, rule);
   const int row = blockIdx.x;  // b * hq + h
   const int b = row / hq;
   const int lane = threadIdx.x;
   const int j = lane >> 5, i = lane & 31;
-  const int L = min(seqlens[b], max_tokens);
+  const int L = min(seqlens[b], rule.max_tokens);
+  const int split_tokens = split_tokens_of(own, L, seqlens, rule);
   const int nvalid = L <= 0 ? 0 : min(splits, (L + split_tokens - 1) / split_tokens);
   if (nvalid == 1) return;
   const float* lse = part_lse + (int64_t)row * splits;
@@ -613,7 +714,9 @@ template <typename T, int S>
 __global__ __launch_bounds__(64) void decode_combine_small_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_lse,
     const int32_t* __restrict__ seqlens, uint16_t* __restrict__ out, int hq,
-    int splits, int split_tokens, int max_tokens) {
+    SplitRule rule) {
+  const int splits = rule.splits;
+  const int own = lane_length(seqlens, rule);
   const int row = blockIdx.x;  // b * hq + h
   const int b = row / hq;
   const int lane = threadIdx.x;
@@ -629,7 +732,8 @@ __global__ __launch_bounds__(64) void decode_combine_small_kernel(
     pv[sp] = sp < splits ? *reinterpret_cast<const float2*>(po + (int64_t)sp * kHeadDim)
                          : float2{0.0f, 0.0f};
   }
-  const int L = min(seqlens[b], max_tokens);
+  const int L = min(seqlens[b], rule.max_tokens);
+  const int split_tokens = split_tokens_of(own, L, seqlens, rule);
   const int nvalid = L <= 0 ? 0 : min(splits, (L + split_tokens - 1) / split_tokens);
   if (nvalid == 1) return;
   float M = -INFINITY;
@@ -666,8 +770,10 @@ constexpr int kWideThreshold = 64;  // splits above this use the wide merge
 template <typename T>
 __global__ __launch_bounds__(64 * kWideWaves) void decode_combine_wide_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_lse,
-    const int32_t* __restrict__ seqlens, uint16_t* __restrict__ out, int hq, int splits,
-    int split_tokens, int max_tokens) {
+    const int32_t* __restrict__ seqlens, uint16_t* __restrict__ out, int hq,
+    SplitRule rule) {
+  const int splits = rule.splits;
+  const int own = lane_length(seqlens, rule);
   __shared__ float s_m[kWideWaves][8], s_den[kWideWaves][8];
   __shared__ __attribute__((aligned(16))) f32x4 s_o[kWideWaves][8];
   const int row = blockIdx.x;  // b * hq + h
@@ -686,7 +792,8 @@ __global__ __launch_bounds__(64 * kWideWaves) void decode_combine_wide_kernel(
   constexpr int kPass = 8 * kWideWaves * kWideK;
   SplitLoads<kWideK> first;
   load_splits(first, lse, po, 8 * wave + j, 8 * kWideWaves, min(splits, kPass));
-  const int L = min(seqlens[b], max_tokens);
+  const int L = min(seqlens[b], rule.max_tokens);
+  const int split_tokens = split_tokens_of(own, L, seqlens, rule);
   const int nvalid = L <= 0 ? 0 : min(splits, (L + split_tokens - 1) / split_tokens);
   if (nvalid == 1) return;  // written by the split kernel
   float m = -INFINITY, den = 0.0f;
@@ -723,19 +830,6 @@ __global__ __launch_bounds__(64 * kWideWaves) void decode_combine_wide_kernel(
 // trip before the writes.
 constexpr int kOrderThreads = 256;
 constexpr int kOrderMaxBatch = 4096;
-
-// Sum over the wave with DPP row shifts and the two cross-row swaps (no
-// LDS round trip).
-__device__ __forceinline__ int wave_sum_i32(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);   // quad_perm [1,0,3,2]
-  v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false);   // quad_perm [2,3,0,1]
-  v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, false);  // row_half_mirror
-  v += __builtin_amdgcn_update_dpp(0, v, 0x140, 0xF, 0xF, false);  // row_mirror
-  const auto r16 = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
-  v = (int)(r16[0] + r16[1]);
-  const auto r32 = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
-  return (int)(r32[0] + r32[1]);
-}
 
 __global__ __launch_bounds__(kOrderThreads) void decode_order_kernel(
     const int32_t* __restrict__ seqlens, const int32_t* __restrict__ bt, int4* __restrict__ items,
@@ -823,8 +917,9 @@ static hipError_t launch_decode(const DecodeArgs& a, int batch, hipStream_t stre
   // with the short sequences last, their longer units no longer lengthen
   // the tail (ragged batch 256: 425-426 against 433-435 us with 4 waves)
   if (wide_wgs <= kWideGridMax || (a.items && units >= kWavesPerWG)) {
-    const dim3 grid((unsigned)((units + kWavesPerWG - 1) / kWavesPerWG), (unsigned)a.splits,
-                    (unsigned)batch);
+    dim3 grid((unsigned)((units + kWavesPerWG - 1) / kWavesPerWG), (unsigned)a.splits,
+              (unsigned)batch);
+    if (a.rule.adapt) std::swap(grid.y, grid.z);
     hipLaunchKernelGGL((decode_fp8_kernel<T, kWavesPerWG>), grid, dim3(64 * kWavesPerWG), 0,
                        stream, a);
   } else {
@@ -838,15 +933,15 @@ static hipError_t launch_decode(const DecodeArgs& a, int batch, hipStream_t stre
   if (a.splits > kWideThreshold)
     hipLaunchKernelGGL(decode_combine_wide_kernel<T>, dim3((unsigned)(batch * a.hq), 4u),
                        dim3(64 * kWideWaves), 0, stream, a.part_o, a.part_lse, a.seqlens, a.out,
-                       a.hq, a.splits, a.pages_per_split * a.bs, a.w * a.bs);
+                       a.hq, a.rule);
   else if (a.splits <= 8)
     hipLaunchKernelGGL((decode_combine_small_kernel<T, 8>), dim3((unsigned)(batch * a.hq)),
                        dim3(64), 0, stream, a.part_o, a.part_lse, a.seqlens, a.out, a.hq,
-                       a.splits, a.pages_per_split * a.bs, a.w * a.bs);
+                       a.rule);
   else
     hipLaunchKernelGGL(decode_combine_kernel<T>, dim3((unsigned)(batch * a.hq)), dim3(64), 0,
-                       stream, a.part_o, a.part_lse, a.seqlens, a.out, a.hq, a.splits,
-                       a.pages_per_split * a.bs, a.w * a.bs);
+                       stream, a.part_o, a.part_lse, a.seqlens, a.out, a.hq,
+                       a.rule);
   return hipGetLastError();
 }
 
@@ -859,7 +954,6 @@ static int pages_per_split_of(int splits, int w) {
 extern "C" int mskv_decode_num_splits(int batch, int num_q_heads,
                                       int num_kv_heads, int max_blocks_per_seq,
                                       int block_size) {
-  (void)block_size;
   if (batch <= 0 || num_kv_heads <= 0 || num_q_heads <= 0 ||
       max_blocks_per_seq <= 0)
     return 1;
@@ -869,7 +963,19 @@ extern "C" int mskv_decode_num_splits(int batch, int num_q_heads,
   int64_t pps = (w * base + mskv::kTargetWaves - 1) / mskv::kTargetWaves;
   if (pps < 1) pps = 1;
   if (pps > mskv::kMaxPagesPerSplit) pps = mskv::kMaxPagesPerSplit;
-  const int64_t splits = (w + pps - 1) / pps;
+  int64_t splits = (w + pps - 1) / pps;
+  // A page per split leaves half the waves idle: finer splits, of two steps at least,
+  // up to two per wave slot (one is expected to run, see split_tokens_of),
+  // as long as the grid and the partials stay small
+  if (splits > 1 && 2 * w * base <= mskv::kTargetWaves && block_size > 0) {
+    const int64_t per = (base / batch + mskv::kWavesPerWG - 1) / mskv::kWavesPerWG * batch;
+    int64_t fine = 2 * mskv::kTargetWaves / base;
+    fine = std::min(fine, (int64_t)w * block_size / (mskv::kMinSplitSteps * mskv::kStep));
+    fine = std::min(fine, mskv::kWideGridMax / per);
+    fine = std::min(fine, (int64_t)(mskv::kFinePartialBytes /
+                                    ((int64_t)batch * num_q_heads * (mskv::kHeadDim + 1) * 4)));
+    splits = std::max(splits, fine);
+  }
   return (int)splits;
 }
 
@@ -952,6 +1058,21 @@ static int decode_checked(const void* query, const void* k_cache, const void* v_
   a.w = max_blocks_per_seq;
   a.splits = num_splits;
   a.pages_per_split = pages_per_split_of(num_splits, max_blocks_per_seq);
+  // Splits follow the lengths on the device where the grid is at most about
+  // two rounds of 8-wave workgroups, one per CU
+  const int64_t per_split = (num_kv_heads * a.qgroups + kWavesPerWG - 1) / kWavesPerWG;
+  const int64_t slots =
+      std::max<int64_t>(256 / per_split - batch / 2, std::max<int64_t>(128 / per_split, 1));
+  // (A page per split is short enough as it is, and up to eight splits are
+  // the shapes whose tables fit the lengths: 64 x 4096 tokens would pay 0.5
+  // us for the same splits.)
+  const bool fine = num_splits > max_blocks_per_seq;
+  const bool adapt = (fine || (a.pages_per_split > 1 && num_splits > 8)) && !a.items &&
+                     batch <= 256 && per_split * num_splits * batch <= kWideGridMax &&
+                     (int64_t)max_blocks_per_seq * block_size <= 1 << 22;
+  a.rule = SplitRule{batch, num_splits, a.pages_per_split * block_size,
+                     max_blocks_per_seq * block_size, adapt, 1.0f / (float)slots,
+                     1.0f / (float)num_splits};
   a.num_blocks = num_blocks;
   a.scale_log2 = softmax_scale * kLog2e;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);

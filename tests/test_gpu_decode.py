@@ -531,3 +531,47 @@ def test_decode_concurrent_streams_match_the_oracle():
         H.assert_attention_close(oa, ref_a)
         H.assert_attention_close(ob, ref_b)
         assert torch.equal(oa, outs_a[0]) and torch.equal(ob, outs_b[0])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hk,lens,width", [
+    # tables far wider than the lengths: the tokens per split follow the
+    # lengths (two 32-token steps at least), so splits end off page borders
+    (32, 8, [63, 64, 65, 1, 0, 127, 128, 129, 255, 257], 64),
+    (32, 8, [4096, 16, 700], 32),
+    # one sequence, splits finer than a page (more of them than table entries)
+    (16, 8, [700], 0), (32, 8, [64 * 7 + 1], 0), (64, 8, [3000], 0),
+    # a batch past the wave's 64 lanes; a group above 16; few kv heads
+    (16, 8, [1 + 37 * i % 400 for i in range(70)], 4), (24, 1, [500, 90], 40),
+    (32, 2, [1000, 31, 2047], 16),
+])
+def test_decode_splits_that_follow_the_lengths(hq, hk, lens, width, dtype):
+    nb = sum((n + H.BLOCK - 1) // H.BLOCK for n in lens) + 2
+    query, tables, caches = _setup(641 + len(lens) + hq, lens, hq, hk, nb, dtype)
+    if width > tables.shape[1]:
+        tables = torch.nn.functional.pad(tables, (0, width - tables.shape[1]), value=-1)
+    _, out = _run_and_check(query, lens, tables, caches)
+    assert all(torch.all(out[i].float() == 0) for i, n in enumerate(lens) if n == 0)
+
+
+def test_decode_splits_follow_the_lengths_of_each_replay():
+    """A captured decode lays its splits out anew from the lengths of every
+    replay: each equals the eager result bit for bit."""
+    lens = [3000, 40, 900, 1500]
+    nb = sum((n + H.BLOCK - 1) // H.BLOCK for n in lens) + 2
+    query, tables, caches = _setup(651, lens, 32, 8, nb)
+    tables = torch.nn.functional.pad(tables, (0, 64 - tables.shape[1]), value=-1).to(H.DEV)
+    q = query.to(H.DEV)
+    static = torch.tensor(lens, dtype=torch.int32, device=H.DEV)
+    out = fp8_decode_attention(q, *caches, static, tables, 0.088)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        fp8_decode_attention(q, *caches, static, tables, 0.088, out=out)
+    for now in (lens, [1, 1, 1, 1], [3000, 0, 0, 0], [65, 40, 900, 1500], [0, 0, 0, 0], lens):
+        static.copy_(torch.tensor(now, dtype=torch.int32))
+        out.fill_(7.0)
+        graph.replay()
+        eager = fp8_decode_attention(q, *caches, static.clone(), tables, 0.088)
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager), now
