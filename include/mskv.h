@@ -66,6 +66,21 @@ int mskv_store_fp8_kvcache(const void* key, const void* value,
                            int64_t num_slots, int act_dtype, void* stream);
 
 /*
+ * mskv_store_fp8_kvcache on keys and values that lie key_stride / value_stride
+ * elements apart from token to token (each at least num_kv_heads * head_dim
+ * and a multiple of 16 bytes, else MSKV_EINVAL): the v view of a qkv
+ * projection needs no copy.  A token's heads are contiguous.
+ */
+int mskv_store_fp8_kvcache_strided(const void* key, int64_t key_stride,
+                                   const void* value, int64_t value_stride,
+                                   void* k_cache, void* v_cache,
+                                   float* k_scale_cache, float* v_scale_cache,
+                                   const void* slot_mapping, int slot_dtype,
+                                   int64_t num_tokens, int num_kv_heads,
+                                   int head_dim, int64_t num_slots,
+                                   int act_dtype, void* stream);
+
+/*
  * Number of split-KV partitions mskv_fp8_decode_attention uses for a shape.
  * Depends on shapes only (never on device sequence lengths), so a captured
  * graph stays valid for any lengths up to max_blocks_per_seq * block_size.
@@ -247,6 +262,23 @@ int mskv_prefill_attention(const void* query, const void* key,
                            int64_t total_q, int64_t total_k, int max_seqlen_q,
                            int num_q_heads, int num_kv_heads, int head_dim,
                            float softmax_scale, int act_dtype, void* stream);
+
+/*
+ * mskv_prefill_attention on keys and values that lie key_stride /
+ * value_stride elements apart from token to token (each at least
+ * num_kv_heads * head_dim and a multiple of 16 bytes, else MSKV_EINVAL; at
+ * most 2^24 - 1, else MSKV_EUNSUPPORTED).  A token's heads are contiguous.
+ */
+int mskv_prefill_attention_strided(const void* query, const void* key,
+                                   int64_t key_stride, const void* value,
+                                   int64_t value_stride, void* out,
+                                   const int32_t* cu_seqlens_q,
+                                   const int32_t* cu_seqlens_k, int num_seqs,
+                                   int64_t total_q, int64_t total_k,
+                                   int max_seqlen_q, int num_q_heads,
+                                   int num_kv_heads, int head_dim,
+                                   float softmax_scale, int act_dtype,
+                                   void* stream);
 
 /*
  * Expand one step's per-sequence scheduling state into its per-token inputs

@@ -30,6 +30,9 @@ _PROTOS = {
     "mskv_store_fp8_kvcache": (_c_int, [
         _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_int,
         _c_i64, _c_int, _c_int, _c_i64, _c_int, _vp]),
+    "mskv_store_fp8_kvcache_strided": (_c_int, [
+        _vp, _c_i64, _vp, _c_i64, _vp, _vp, _vp, _vp, _vp, _c_int,
+        _c_i64, _c_int, _c_int, _c_i64, _c_int, _vp]),
     "mskv_decode_num_splits": (_c_int, [_c_int, _c_int, _c_int, _c_int, _c_int]),
     "mskv_decode_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int, _c_int, _c_int]),
     "mskv_fp8_decode_attention": (_c_int, [
@@ -52,6 +55,9 @@ _PROTOS = {
         _c_int, _c_f32, _c_int, _vp, _c_size, _vp]),
     "mskv_prefill_attention": (_c_int, [
         _vp, _vp, _vp, _vp, _vp, _vp, _c_int, _c_i64, _c_i64, _c_int,
+        _c_int, _c_int, _c_int, _c_f32, _c_int, _vp]),
+    "mskv_prefill_attention_strided": (_c_int, [
+        _vp, _vp, _c_i64, _vp, _c_i64, _vp, _vp, _vp, _c_int, _c_i64, _c_i64, _c_int,
         _c_int, _c_int, _c_int, _c_f32, _c_int, _vp]),
     "mskv_build_step_inputs": (_c_int, [
         _vp, _vp, _vp, _vp, _vp, _c_int, _c_int, _c_i64, _c_int, _c_int, _c_i64,
@@ -110,6 +116,23 @@ def store_dtype(t) -> int:
     if t.dtype in (torch.float16, torch.bfloat16):
         return act_dtype(t)
     raise AssertionError(f"key/value dtype must be float16, bfloat16 or float32, got {t.dtype}")
+
+
+def token_rows(t):
+    """A ``[tokens, heads, D]`` tensor and the elements between its tokens,
+    for a kernel that reads whole tokens at any stride: a view with each
+    token's heads together (the v view of a qkv projection) as it is, if its
+    rows start on 16 bytes and the stride fits the kernels' 32-bit tile
+    offsets; anything else as a contiguous copy."""
+    heads, d = t.shape[1], t.shape[2]
+    if not t.is_contiguous():
+        s0, s1, s2 = t.stride()
+        size = t.element_size()
+        if (s2 == 1 and s1 == d and heads * d <= s0 <= 1 << 22 and s0 * size % 16 == 0
+                and t.data_ptr() % 16 == 0):
+            return t, s0
+        t = t.contiguous()
+    return t, heads * d
 
 
 def on_device(what: str, ref, *tensors) -> None:

@@ -41,6 +41,8 @@
 //    grid.
 #include <math.h>
 
+#include <algorithm>
+
 #include "mskv_device.h"
 #include "../../include/mskv.h"
 
@@ -72,6 +74,7 @@ struct DenseArgs {
   const int32_t* cu_q;
   const int32_t* cu_k;
   int64_t total_q, total_k;
+  int64_t k_stride, v_stride;  // elements between the tokens of key / value
   int hq, hk, group, gc, qgroups, tpr;
   float scale_log2;
 };
@@ -178,22 +181,23 @@ __global__ __launch_bounds__(kDThreads, 2) void dense_prefill_kernel(DenseArgs a
   const uint32_t v_row = (uint32_t)(4 * g + (sl >> 2)) * kDRow + 8u * (uint32_t)(sl & 1);
   const uint32_t v_x = 16u * (uint32_t)(((sl & 3) >> 1) ^ (4 * g + (sl >> 2)));
 
-  const uint32_t rstride = (uint32_t)a.hk * kDRow;  // bytes between key rows
+  // bytes between key / value rows
+  const uint32_t k_rstride = 2u * (uint32_t)a.k_stride, v_rstride = 2u * (uint32_t)a.v_stride;
   auto stage_tile = [&](int t0, uint8_t* kt, uint8_t* vt) {
     const int valid = min(kDStep, lk - t0);
-    const int64_t e0 = ((k_begin + t0) * a.hk + kvh) * kHeadDim;
-    const uint32_t bytes = valid > 0 ? (uint32_t)(valid - 1) * rstride + kDRow : 0u;
-    const auto kr = make_rsrc(a.k + e0, bytes);
-    const auto vr = make_rsrc(a.v + e0, bytes);
+    const int64_t row = k_begin + t0, head = (int64_t)kvh * kHeadDim;
+    const auto kr = make_rsrc(a.k + row * a.k_stride + head,
+                              valid > 0 ? (uint32_t)(valid - 1) * k_rstride + kDRow : 0u);
+    const auto vr = make_rsrc(a.v + row * a.v_stride + head,
+                              valid > 0 ? (uint32_t)(valid - 1) * v_rstride + kDRow : 0u);
     // wave w's j-th load fills rows 4(4j + w) .. +4: lane i lands in slot i,
     // i.e. row 4(4j + w) + i/16 at swizzled position i%16
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int row = 4 * (4 * j + wave) + (lane >> 4);
       const int c = (lane & 15) ^ (row & 15);
-      const uint32_t o = (uint32_t)row * rstride + 16u * (uint32_t)c;
-      lds_load16_d(kr, kt + 1024 * (4 * j + wave), o);
-      lds_load16_d(vr, vt + 1024 * (4 * j + wave), o);
+      lds_load16_d(kr, kt + 1024 * (4 * j + wave), (uint32_t)row * k_rstride + 16u * (uint32_t)c);
+      lds_load16_d(vr, vt + 1024 * (4 * j + wave), (uint32_t)row * v_rstride + 16u * (uint32_t)c);
     }
   };
 
@@ -401,12 +405,11 @@ static hipError_t launch_dense_sized(const DenseArgs& a, int num_seqs, int max_s
 
 }  // namespace mskv
 
-extern "C" int mskv_prefill_attention(const void* query, const void* key, const void* value,
-                                      void* out, const int32_t* cu_seqlens_q,
-                                      const int32_t* cu_seqlens_k, int num_seqs,
-                                      int64_t total_q, int64_t total_k, int max_seqlen_q,
-                                      int num_q_heads, int num_kv_heads, int head_dim,
-                                      float softmax_scale, int act_dtype, void* stream) {
+extern "C" int mskv_prefill_attention_strided(
+    const void* query, const void* key, int64_t key_stride, const void* value,
+    int64_t value_stride, void* out, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+    int num_seqs, int64_t total_q, int64_t total_k, int max_seqlen_q, int num_q_heads,
+    int num_kv_heads, int head_dim, float softmax_scale, int act_dtype, void* stream) {
   if (num_seqs < 0 || total_q < 0 || total_k < 0 || max_seqlen_q < 0 || num_q_heads <= 0 ||
       num_kv_heads <= 0)
     return MSKV_EINVAL;
@@ -417,10 +420,16 @@ extern "C" int mskv_prefill_attention(const void* query, const void* key, const 
   // the row maxima are taken before the scale, which must keep their order
   const float scale_log2 = softmax_scale * mskv::kLog2e;
   if (!(scale_log2 > 0.0f && scale_log2 < INFINITY)) return MSKV_EUNSUPPORTED;
+  // rows start on 16 bytes
+  const int64_t kv_row = (int64_t)num_kv_heads * head_dim;
+  if (key_stride < kv_row || value_stride < kv_row || key_stride % 8 != 0 ||
+      value_stride % 8 != 0)
+    return MSKV_EINVAL;
   if (num_seqs == 0 || total_q == 0 || max_seqlen_q == 0) return MSKV_OK;
   if (!query || !key || !value || !out || !cu_seqlens_q || !cu_seqlens_k) return MSKV_EINVAL;
-  // per-tile offsets are 32-bit: 64 key rows of all kv heads
-  if ((int64_t)mskv::kDStep * num_kv_heads * mskv::kDRow > 0x7FFFFFFFLL) return MSKV_EUNSUPPORTED;
+  // per-tile offsets are 32-bit: 64 key rows
+  if (std::max(key_stride, value_stride) > 0x7FFFFFFFLL / (2 * mskv::kDStep))
+    return MSKV_EUNSUPPORTED;
 
   mskv::DenseArgs a;
   a.q = (const uint16_t*)query;
@@ -431,6 +440,8 @@ extern "C" int mskv_prefill_attention(const void* query, const void* key, const 
   a.cu_k = cu_seqlens_k;
   a.total_q = total_q;
   a.total_k = total_k;
+  a.k_stride = key_stride;
+  a.v_stride = value_stride;
   a.hq = num_q_heads;
   a.hk = num_kv_heads;
   a.group = group;
@@ -446,4 +457,17 @@ extern "C" int mskv_prefill_attention(const void* query, const void* key, const 
   if (act_dtype == MSKV_BFLOAT16)
     return (int)mskv::launch_dense_sized<__bf16>(a, num_seqs, max_seqlen_q, st);
   return (int)mskv::launch_dense_sized<_Float16>(a, num_seqs, max_seqlen_q, st);
+}
+
+extern "C" int mskv_prefill_attention(const void* query, const void* key, const void* value,
+                                      void* out, const int32_t* cu_seqlens_q,
+                                      const int32_t* cu_seqlens_k, int num_seqs,
+                                      int64_t total_q, int64_t total_k, int max_seqlen_q,
+                                      int num_q_heads, int num_kv_heads, int head_dim,
+                                      float softmax_scale, int act_dtype, void* stream) {
+  const int64_t row = (int64_t)num_kv_heads * head_dim;
+  return mskv_prefill_attention_strided(query, key, row, value, row, out, cu_seqlens_q,
+                                        cu_seqlens_k, num_seqs, total_q, total_k, max_seqlen_q,
+                                        num_q_heads, num_kv_heads, head_dim, softmax_scale,
+                                        act_dtype, stream);
 }

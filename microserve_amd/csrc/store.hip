@@ -20,14 +20,14 @@ constexpr int kStoreLanesPerRow = kHeadDim / 16;  // 8
 constexpr int kStoreThreads = 256;
 constexpr int kStoreRowsPerBlock = kStoreThreads / kStoreLanesPerRow;
 
-// This lane's 16 elements of row `row` as fp32 (streaming loads: each row
-// is read once).  16-bit inputs convert exactly; fp32 inputs are used as
-// they are, as the reference's upcast leaves them.
+// This lane's 16 elements of the row that starts at element `at`, as fp32
+// (streaming loads: each row is read once).  16-bit inputs convert exactly;
+// fp32 inputs are used as they are, as the reference's upcast leaves them.
 template <typename T>
-__device__ __forceinline__ void load16(const void* base, int64_t row, int sub, float* x) {
+__device__ __forceinline__ void load16(const void* base, int64_t at, int sub, float* x) {
   if constexpr (sizeof(T) == 4) {
     const u32x4* p = reinterpret_cast<const u32x4*>(
-        reinterpret_cast<const float*>(base) + row * kHeadDim + sub * 16);
+        reinterpret_cast<const float*>(base) + at + sub * 16);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       const u32x4 v = __builtin_nontemporal_load(p + c);
@@ -36,7 +36,7 @@ __device__ __forceinline__ void load16(const void* base, int64_t row, int sub, f
     }
   } else {
     const u32x4* p = reinterpret_cast<const u32x4*>(
-        reinterpret_cast<const uint16_t*>(base) + row * kHeadDim + sub * 16);
+        reinterpret_cast<const uint16_t*>(base) + at + sub * 16);
     const u32x4 a = __builtin_nontemporal_load(p);
     const u32x4 b = __builtin_nontemporal_load(p + 1);
 #pragma unroll
@@ -49,13 +49,15 @@ __device__ __forceinline__ void load16(const void* base, int64_t row, int sub, f
   }
 }
 
-template <typename T, typename SlotT>
+// kPacked: both inputs are contiguous, so a row's number is its place
+// (the 262,144-token fill: 296 us, 298 with two strides)
+template <typename T, typename SlotT, bool kPacked>
 __global__ __launch_bounds__(kStoreThreads) void store_fp8_kernel(
     const void* __restrict__ key, const void* __restrict__ value,
     uint8_t* __restrict__ k_cache, uint8_t* __restrict__ v_cache,
     float* __restrict__ k_scale, float* __restrict__ v_scale,
     const SlotT* __restrict__ slots, int64_t rows, int num_kv_heads,
-    int64_t num_slots) {
+    int64_t num_slots, int64_t key_stride, int64_t value_stride) {
   const int sub = threadIdx.x % kStoreLanesPerRow;
   const int64_t row =
       (int64_t)blockIdx.x * kStoreRowsPerBlock + threadIdx.x / kStoreLanesPerRow;
@@ -64,11 +66,13 @@ __global__ __launch_bounds__(kStoreThreads) void store_fp8_kernel(
   const int head = (int)(row - tok * num_kv_heads);
   const int64_t slot = (int64_t)slots[tok];
 
+  // Tokens may lie apart (the v view of a qkv projection): the copy that
+  // would pack them costs a launch, 4 to 5 us on a decode step or a chunk.
   float x[16];
   u32x4 kq, vq;
-  load16<T>(key, row, sub, x);
+  load16<T>(key, kPacked ? row * kHeadDim : tok * key_stride + head * kHeadDim, sub, x);
   const float ks = quantize16(x, kq);
-  load16<T>(value, row, sub, x);
+  load16<T>(value, kPacked ? row * kHeadDim : tok * value_stride + head * kHeadDim, sub, x);
   const float vs = quantize16(x, vq);
 
   if (slot < 0 || slot >= num_slots) return;
@@ -89,35 +93,45 @@ static hipError_t launch_store(const void* key, const void* value, void* kc,
                                void* vc, float* ks, float* vs,
                                const void* slots, int slot_dtype,
                                int64_t num_tokens, int hk, int64_t num_slots,
-                               hipStream_t stream) {
+                               int64_t key_stride, int64_t value_stride, hipStream_t stream) {
   const int64_t rows = num_tokens * hk;
   const int64_t blocks = (rows + kStoreRowsPerBlock - 1) / kStoreRowsPerBlock;
-  if (slot_dtype == MSKV_INT64)
-    hipLaunchKernelGGL((store_fp8_kernel<T, int64_t>), dim3((unsigned)blocks),
-                       dim3(kStoreThreads), 0, stream, key, value, (uint8_t*)kc,
-                       (uint8_t*)vc, ks, vs, (const int64_t*)slots, rows, hk, num_slots);
-  else
-    hipLaunchKernelGGL((store_fp8_kernel<T, int32_t>), dim3((unsigned)blocks),
-                       dim3(kStoreThreads), 0, stream, key, value, (uint8_t*)kc,
-                       (uint8_t*)vc, ks, vs, (const int32_t*)slots, rows, hk, num_slots);
+  auto launch = [&](auto kernel, auto* typed_slots) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kStoreThreads), 0, stream, key, value,
+                       (uint8_t*)kc, (uint8_t*)vc, ks, vs, typed_slots, rows, hk, num_slots,
+                       key_stride, value_stride);
+  };
+  const bool packed = key_stride == (int64_t)hk * kHeadDim && value_stride == key_stride;
+  if (slot_dtype == MSKV_INT64) {
+    const auto* p = (const int64_t*)slots;
+    packed ? launch(store_fp8_kernel<T, int64_t, true>, p)
+           : launch(store_fp8_kernel<T, int64_t, false>, p);
+  } else {
+    const auto* p = (const int32_t*)slots;
+    packed ? launch(store_fp8_kernel<T, int32_t, true>, p)
+           : launch(store_fp8_kernel<T, int32_t, false>, p);
+  }
   return hipGetLastError();
 }
 
 }  // namespace mskv
 
-extern "C" int mskv_store_fp8_kvcache(const void* key, const void* value,
-                                      void* k_cache, void* v_cache,
-                                      float* k_scale_cache,
-                                      float* v_scale_cache,
-                                      const void* slot_mapping, int slot_dtype,
-                                      int64_t num_tokens, int num_kv_heads,
-                                      int head_dim, int64_t num_slots,
-                                      int act_dtype, void* stream) {
+extern "C" int mskv_store_fp8_kvcache_strided(
+    const void* key, int64_t key_stride, const void* value, int64_t value_stride, void* k_cache,
+    void* v_cache, float* k_scale_cache, float* v_scale_cache, const void* slot_mapping,
+    int slot_dtype, int64_t num_tokens, int num_kv_heads, int head_dim, int64_t num_slots,
+    int act_dtype, void* stream) {
   if (num_tokens < 0 || num_kv_heads <= 0 || num_slots < 0) return MSKV_EINVAL;
   if (slot_dtype != MSKV_INT32 && slot_dtype != MSKV_INT64) return MSKV_EINVAL;
   if (act_dtype != MSKV_FLOAT16 && act_dtype != MSKV_BFLOAT16 && act_dtype != MSKV_FLOAT32)
     return MSKV_EINVAL;
   if (head_dim != mskv::kHeadDim) return MSKV_EUNSUPPORTED;
+  // rows start on 16 bytes
+  const int64_t row = (int64_t)num_kv_heads * head_dim;
+  const int64_t unit = act_dtype == MSKV_FLOAT32 ? 4 : 8;
+  if (key_stride < row || value_stride < row || key_stride % unit != 0 ||
+      value_stride % unit != 0)
+    return MSKV_EINVAL;
   if (num_tokens == 0) return MSKV_OK;
   if (!key || !value || !k_cache || !v_cache || !k_scale_cache ||
       !v_scale_cache || !slot_mapping)
@@ -130,14 +144,28 @@ extern "C" int mskv_store_fp8_kvcache(const void* key, const void* value,
   if (act_dtype == MSKV_BFLOAT16)
     e = mskv::launch_store<__bf16>(key, value, k_cache, v_cache, k_scale_cache, v_scale_cache,
                                    slot_mapping, slot_dtype, num_tokens, num_kv_heads,
-                                   num_slots, s);
+                                   num_slots, key_stride, value_stride, s);
   else if (act_dtype == MSKV_FLOAT16)
     e = mskv::launch_store<_Float16>(key, value, k_cache, v_cache, k_scale_cache,
                                      v_scale_cache, slot_mapping, slot_dtype, num_tokens,
-                                     num_kv_heads, num_slots, s);
+                                     num_kv_heads, num_slots, key_stride, value_stride, s);
   else
     e = mskv::launch_store<float>(key, value, k_cache, v_cache, k_scale_cache, v_scale_cache,
                                   slot_mapping, slot_dtype, num_tokens, num_kv_heads,
-                                  num_slots, s);
+                                  num_slots, key_stride, value_stride, s);
   return (int)e;
+}
+
+extern "C" int mskv_store_fp8_kvcache(const void* key, const void* value,
+                                      void* k_cache, void* v_cache,
+                                      float* k_scale_cache,
+                                      float* v_scale_cache,
+                                      const void* slot_mapping, int slot_dtype,
+                                      int64_t num_tokens, int num_kv_heads,
+                                      int head_dim, int64_t num_slots,
+                                      int act_dtype, void* stream) {
+  const int64_t row = (int64_t)num_kv_heads * head_dim;
+  return mskv_store_fp8_kvcache_strided(key, row, value, row, k_cache, v_cache, k_scale_cache,
+                                        v_scale_cache, slot_mapping, slot_dtype, num_tokens,
+                                        num_kv_heads, head_dim, num_slots, act_dtype, stream);
 }

@@ -25,8 +25,6 @@ def store_fp8_kvcache(
     reference upcasts any float to fp32, ``:22-23``); ``slot_mapping`` may be
     int32 or int64.
     """
-    key = key.contiguous()
-    value = value.contiguous()
     slot_mapping = slot_mapping.contiguous()
     num_tokens, num_kv_heads, head_dim = key.shape
     assert value.shape == key.shape
@@ -43,10 +41,12 @@ def store_fp8_kvcache(
         assert t.is_contiguous(), "caches must be contiguous"
     _lib.on_device("store_fp8_kvcache", key, value, k_cache, v_cache, k_scale_cache,
                    v_scale_cache, slot_mapping)
+    key, key_stride = _lib.token_rows(key)
+    value, value_stride = _lib.token_rows(value)
     num_slots = k_cache.shape[0] * k_cache.shape[1]
     lib = _lib.load()
-    status = lib.mskv_store_fp8_kvcache(
-        key.data_ptr(), value.data_ptr(), k_cache.data_ptr(),
+    status = lib.mskv_store_fp8_kvcache_strided(
+        key.data_ptr(), key_stride, value.data_ptr(), value_stride, k_cache.data_ptr(),
         v_cache.data_ptr(), k_scale_cache.data_ptr(), v_scale_cache.data_ptr(),
         slot_mapping.data_ptr(),
         _lib.INT64 if slot_mapping.dtype == torch.int64 else _lib.INT32,

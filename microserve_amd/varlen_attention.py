@@ -31,8 +31,6 @@ def varlen_attention(
     del max_seqlen_k
     assert causal, "only causal attention is provided (the path never calls it otherwise)"
     q = q.contiguous()
-    k = k.contiguous()
-    v = v.contiguous()
     cu_seqlens_q = cu_seqlens_q.contiguous()
     cu_seqlens_k = cu_seqlens_k.contiguous()
     total_q, num_q_heads, head_dim = q.shape
@@ -45,14 +43,16 @@ def varlen_attention(
     num_seqs = cu_seqlens_q.numel() - 1
     assert cu_seqlens_k.numel() == num_seqs + 1
     _lib.on_device("varlen_attention", q, k, v, cu_seqlens_q, cu_seqlens_k)
+    k, k_stride = _lib.token_rows(k)
+    v, v_stride = _lib.token_rows(v)
     if softmax_scale is None:
         softmax_scale = head_dim ** -0.5
     out = torch.empty_like(q)
     if total_q == 0 or num_seqs == 0:
         return out
     lib = _lib.load()
-    status = lib.mskv_prefill_attention(
-        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+    status = lib.mskv_prefill_attention_strided(
+        q.data_ptr(), k.data_ptr(), k_stride, v.data_ptr(), v_stride, out.data_ptr(),
         cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(), num_seqs,
         total_q, total_k, int(max_seqlen_q), num_q_heads, num_kv_heads,
         head_dim, float(softmax_scale), _lib.act_dtype(q), _lib.stream_of(q))

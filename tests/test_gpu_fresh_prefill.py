@@ -145,3 +145,23 @@ def test_fresh_prefill_random_shapes(case):
 def test_fresh_prefill_block_sizes_at_their_edges(hq, hk, lens, dtype):
     q, k, v, cu_q, cu_k = _setup(451 + sum(lens), lens, lens, hq, hk, dtype)
     _check(q, k, v, cu_q, cu_k, lens, lens)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_fresh_prefill_reads_strided_tokens_like_their_copies(dtype):
+    """k and v as views of wider rows (each its own stride), and forms that
+    the kernel cannot read in place, give the contiguous copies' bits."""
+    gen = torch.Generator().manual_seed(461)
+    lens, hk = [130, 1, 65], 8
+    n = sum(lens)
+    cu = torch.tensor([0, 130, 131, 196], dtype=torch.int32, device=H.DEV)
+    q = torch.randn(n, 32, H.D, generator=gen).to(dtype).to(H.DEV)
+    kw = torch.randn(n, (hk + 1) * H.D, generator=gen).to(dtype).to(H.DEV)
+    vw = torch.randn(n, 3 * hk * H.D, generator=gen).to(dtype).to(H.DEV)
+    views = [(kw[:, :hk * H.D].view(n, hk, H.D), vw[:, 2 * hk * H.D:].view(n, hk, H.D)),
+             (kw[:, 4:4 + hk * H.D].view(n, hk, H.D), vw.view(n, 3 * hk, H.D)[:, ::3])]
+    for k, v in views:
+        got = varlen_attention(q, k, v, cu, cu, max(lens), max(lens))
+        want = varlen_attention(q, k.contiguous(), v.contiguous(), cu, cu, max(lens), max(lens))
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)

@@ -188,3 +188,30 @@ def test_store_fill_qwen3_8b_pool_sampled_and_roundtrip():
     assert used.sum() == 1024
     free = (~used).nonzero().view(-1).to(H.DEV)
     assert (kc.view(torch.uint8)[free] == 0).all() and (ks[free] == 1).all()
+
+
+def _token_views(gen, n, hk, dtype):
+    """[n, hk, D] views of one matrix of wider rows, and forms that are not
+    whole tokens on 16 bytes (offset, head order, expanded, one token)."""
+    wide = torch.randn(n, 3 * hk * H.D + 8, generator=gen).to(dtype).to(H.DEV)
+    yield "view", wide[:, hk * H.D:2 * hk * H.D].view(n, hk, H.D)
+    yield "off 16 bytes", wide[:, 1:1 + hk * H.D].view(n, hk, H.D)
+    yield "heads apart", wide[:, :2 * hk * H.D].view(n, hk, 2 * H.D)[..., :H.D]
+    yield "heads first", wide[:, :hk * H.D].contiguous().view(hk, n, H.D).transpose(0, 1)
+    yield "expanded", wide[:1, :hk * H.D].view(1, hk, H.D).expand(n, hk, H.D)
+    yield "every other token", wide[::2, :hk * H.D].repeat(2, 1)[:n].view(n, hk, H.D)
+    yield "odd row length", wide[:, :3 * hk * H.D + 7][:, :hk * H.D].view(n, hk, H.D)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("n,hk", [(1, 8), (33, 8), (5, 1)])
+def test_store_reads_strided_tokens_like_their_copies(n, hk, dtype):
+    gen = torch.Generator().manual_seed(71 + n)
+    slots = torch.randperm(4 * H.BLOCK, generator=gen)[:n].to(H.DEV)
+    for name, view in _token_views(gen, n, hk, dtype):
+        for key, value in ((view, view.contiguous()), (view.contiguous(), view), (view, view)):
+            a, b = H.alloc_cache(4, H.BLOCK, hk), H.alloc_cache(4, H.BLOCK, hk)
+            store_fp8_kvcache(key, value, *a, slots)
+            store_fp8_kvcache(key.contiguous(), value.contiguous(), *b, slots)
+            for x, y in zip(a, b):
+                assert torch.equal(x.view(torch.uint8), y.view(torch.uint8)), name
