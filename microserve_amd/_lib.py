@@ -11,6 +11,20 @@ from __future__ import annotations
 import ctypes
 import os
 
+import torch  # noqa: F401  (the extension below uses its libraries)
+
+try:
+    from microserve_amd import _fast_calls as fast
+except ImportError as e:  # raised on use: the package must import to be built
+    class _NotBuilt:
+        why = e
+
+        def __getattr__(self, name):
+            raise RuntimeError("microserve_amd._fast_calls is not built: run "
+                               f"`python -m microserve_amd.build` ({self.why})")
+
+    fast = _NotBuilt()
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libmskv.so")
 
@@ -87,6 +101,7 @@ def load() -> ctypes.CDLL:
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
+    fast.bind({name: ctypes.cast(getattr(lib, name), _vp).value for name in _PROTOS})
     _lib = lib
     return lib
 

@@ -2,7 +2,9 @@
 
 Compiles every source under ``csrc/`` with hipcc into
 ``microserve_amd/libmskv.so``, and ``csrc/host/step_pack.cpp`` with g++
-into the ``microserve_amd._step_pack`` extension module.  Run ``python -m microserve_amd.build``.
+into the ``microserve_amd._step_pack`` extension module, and
+``csrc/host/fast_calls.cpp`` (which uses torch's headers) into
+``microserve_amd._fast_calls``.  Run ``python -m microserve_amd.build``.
 The library is built in-tree so it travels with the repository snapshot.
 """
 
@@ -21,6 +23,9 @@ ARCH = "gfx950"
 # the host packer of the step-input builder, a CPython extension module
 PACK_SRC = os.path.join(CSRC, "host", "step_pack.cpp")
 PACK_OUT = os.path.join(HERE, "_step_pack" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
+# the native call paths of the hot entry points, against torch's libraries
+FAST_SRC = os.path.join(CSRC, "host", "fast_calls.cpp")
+FAST_OUT = os.path.join(HERE, "_fast_calls" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
 
 # -packed-fp32-ops: keep hipcc from emitting v_pk_{add,mul,fma}_f32.
 # No fast-math: the store path relies on hipcc's correctly rounded fp32
@@ -82,6 +87,7 @@ def build(verbose: bool = False) -> str:
         raise RuntimeError(f"link failed:\n{r.stderr}")
     os.replace(tmp_out, OUT)
     build_pack(verbose)
+    build_fast(verbose)
     return OUT
 
 
@@ -98,6 +104,32 @@ def build_pack(verbose: bool = False) -> str:
         raise RuntimeError(f"g++ failed on {PACK_SRC}:\n{r.stderr}")
     os.replace(tmp_out, PACK_OUT)
     return PACK_OUT
+
+
+def build_fast(verbose: bool = False) -> str:
+    """Compile the native call paths (host C++, torch's headers) with g++."""
+    import torch
+    root = os.path.dirname(torch.__file__)
+    inc = os.path.join(root, "include")
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(shutil.which("hipcc")
+                                                            or "/opt/rocm/bin/hipcc")))
+    cxx = shutil.which("g++") or "g++"
+    tmp_out = FAST_OUT + ".tmp"
+    cmd = [cxx, "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-Wno-unknown-pragmas",
+           "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-isystem", inc, "-isystem", os.path.join(inc, "torch", "csrc", "api", "include"),
+           "-isystem", os.path.join(rocm, "include"),
+           "-I" + sysconfig.get_paths()["include"], FAST_SRC, "-o", tmp_out,
+           "-L" + os.path.join(root, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch",
+           "-ltorch_python"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on {FAST_SRC}:\n{r.stderr}")
+    os.replace(tmp_out, FAST_OUT)
+    return FAST_OUT
 
 
 if __name__ == "__main__":

@@ -66,6 +66,10 @@ def fp8_chunk_prefill_attention(
     bits for every weight.
     """
     del block_m, block_n
+    res = _lib.fast.prefill(query, k_cache, v_cache, k_scale_cache, v_scale_cache, block_table,
+                              None, None, prefix_len, 0, softmax_scale)
+    if res is not None:
+        return res
     query = query.contiguous()
     block_table = block_table.contiguous().view(-1)
     query_len = query.shape[0]
@@ -99,6 +103,10 @@ def fp8_varlen_prefill_attention(
     ``block_tables`` is int32 ``[num_seqs, max_blocks]``.  ``max_seqlen_q``
     is a host integer, as in the reference's ``Context``.
     """
+    res = _lib.fast.prefill(query, k_cache, v_cache, k_scale_cache, v_scale_cache, block_tables,
+                              cu_seqlens_q, cu_seqlens_k, 0, max_seqlen_q, softmax_scale)
+    if res is not None:
+        return res
     query = query.contiguous()
     block_tables = block_tables.contiguous()
     cu_seqlens_q = cu_seqlens_q.contiguous()

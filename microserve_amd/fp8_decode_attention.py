@@ -79,6 +79,10 @@ def fp8_decode_attention(
     ``out``, when given, receives the result instead of a new tensor.
     """
     del block_n
+    res = _lib.fast.decode(query, k_cache, v_cache, k_scale_cache, v_scale_cache, cache_seqlens,
+                             block_tables, softmax_scale, out, _scratch)
+    if res is not None:
+        return res
     query = query.contiguous()
     cache_seqlens = cache_seqlens.contiguous()
     block_tables = block_tables.contiguous()

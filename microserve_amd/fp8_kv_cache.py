@@ -25,6 +25,9 @@ def store_fp8_kvcache(
     reference upcasts any float to fp32, ``:22-23``); ``slot_mapping`` may be
     int32 or int64.
     """
+    if _lib.fast.store(key, value, k_cache, v_cache, k_scale_cache, v_scale_cache,
+                         slot_mapping):
+        return
     slot_mapping = slot_mapping.contiguous()
     num_tokens, num_kv_heads, head_dim = key.shape
     assert value.shape == key.shape

@@ -37,6 +37,11 @@ def qk_norm_rope_store(positions, q, k, v, q_norm_weight, k_norm_weight, eps,
     outside the rotary tables gets zero outputs and is not stored (the
     reference's table lookup would raise there).
     """
+    res = _lib.fast.prologue(positions, q, k, v, q_norm_weight, k_norm_weight, eps, cos_cache,
+                               sin_cache, k_cache, v_cache, k_scale_cache, v_scale_cache,
+                               slot_mapping, return_k)
+    if res is not None:
+        return res
     assert q.dim() == 3 and k.dim() == 3 and v.dim() == 3
     n, hq, d = q.shape
     hk = k.shape[1]

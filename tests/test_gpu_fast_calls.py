@@ -1,0 +1,117 @@
+"""The native call paths take ordinary calls, give the wrappers' own results
+bit for bit, and leave everything else to the wrappers."""
+
+import pytest
+import torch
+
+from tests import gpu_helpers as H
+
+pytestmark = pytest.mark.gpu
+
+from microserve_amd import (_lib, fp8_chunk_prefill_attention, fp8_decode_attention,  # noqa: E402
+                            fp8_varlen_prefill_attention, qk_norm_rope_store, store_fp8_kvcache,
+                            varlen_attention)
+
+
+class _Off:
+    """Native paths that take nothing: the wrappers' own."""
+
+    def __getattr__(self, name):
+        return lambda *a: None
+
+
+def _both(monkeypatch, call):
+    _lib.load()
+    fast = call()
+    with monkeypatch.context() as m:
+        m.setattr(_lib, "fast", _Off())
+        slow = call()
+    torch.cuda.synchronize()
+    for a, b in zip(fast, slow):
+        assert (a is None and b is None) or torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+    return fast
+
+
+def _case(dtype, n=5, hq=8, hk=2, blocks=6):
+    gen = torch.Generator().manual_seed(811)
+    qkv = torch.randn(n, (hq + 2 * hk) * H.D, generator=gen).to(dtype).to(H.DEV)
+    q, k, v = (t.view(n, -1, H.D) for t in qkv.split((hq * H.D, hk * H.D, hk * H.D), -1))
+    slots = torch.randperm(blocks * H.BLOCK, generator=gen)[:n].to(H.DEV)
+    return q, k, v, slots, H.alloc_cache(blocks, H.BLOCK, hk)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_native_paths_give_the_wrappers_results(dtype, monkeypatch):
+    q, k, v, slots, caches = _case(dtype)
+    n = q.shape[0]
+
+    def store():
+        c = H.alloc_cache(6, H.BLOCK, 2)
+        store_fp8_kvcache(k.contiguous(), v, *c, slots)
+        return c
+
+    caches = _both(monkeypatch, store)
+    qc = q.contiguous()
+    lens = torch.tensor([300, 1, 0, 256, 40], dtype=torch.int32, device=H.DEV)
+    tables = torch.tensor([[0, 1], [2, -1], [-1, -1], [3, -1], [4, 5]], dtype=torch.int32,
+                          device=H.DEV)
+    out = torch.empty_like(qc)
+    _both(monkeypatch, lambda: [fp8_decode_attention(qc, *caches, lens, tables, 0.1)])
+    (got,) = _both(monkeypatch,
+                   lambda: [fp8_decode_attention(qc, *caches, lens, tables, 0.1, out=out)])
+    assert got is out
+    _both(monkeypatch, lambda: [fp8_chunk_prefill_attention(qc, *caches, tables[:1], 200, 0.1)])
+    cu = torch.tensor([0, 2, n], dtype=torch.int32, device=H.DEV)
+    ck = torch.tensor([0, 300, 500], dtype=torch.int32, device=H.DEV)
+    _both(monkeypatch, lambda: [fp8_varlen_prefill_attention(qc, *caches, tables[:2], cu, ck, 3,
+                                                             0.1)])
+    for kk in (k, k.contiguous()):
+        _both(monkeypatch, lambda: [varlen_attention(qc, kk, v, cu, cu, 3)])
+    cos, sin = (torch.randn(64, 1, H.D, device=H.DEV).to(dtype) for _ in range(2))
+    w = torch.randn(H.D, device=H.DEV).to(dtype)
+    pos = torch.arange(n, device=H.DEV)
+    for weight in (w, None):
+        for return_k in (True, False):
+            def prologue():
+                c = H.alloc_cache(6, H.BLOCK, 2)
+                return [*qk_norm_rope_store(pos, q, k, v, weight, weight, 1e-6, cos, sin, *c,
+                                            slots, return_k=return_k), *c]
+            _both(monkeypatch, prologue)
+
+
+def test_native_paths_leave_the_rest_to_the_wrappers():
+    q, k, v, slots, caches = _case(torch.float16)
+    _lib.load()
+    lens = torch.ones(5, dtype=torch.int32, device=H.DEV)
+    tables = torch.zeros(5, 1, dtype=torch.int32, device=H.DEV)
+
+    def taken(q=q.contiguous(), caches=caches, lens=lens, tables=tables, scale=0.1, out=None):
+        from microserve_amd.fp8_decode_attention import _scratch
+        return _lib.fast.decode(q, *caches, lens, tables, scale, out, _scratch) is not None
+
+    class Sub(torch.Tensor):
+        pass
+
+    assert taken()
+    assert not taken(q=q)                                       # a strided query
+    assert not taken(q=q.contiguous().as_subclass(Sub))
+    assert not taken(q=q.contiguous().float())
+    assert not taken(lens=lens.long()) and not taken(lens=lens[:4]) and not taken(lens=lens.cpu())
+    assert not taken(tables=tables.view(-1)) and not taken(tables=tables.expand(5, 2))
+    assert not taken(caches=[caches[0].transpose(0, 1), *caches[1:]])
+    assert not taken(scale="0.1") and not taken(out=torch.empty_like(q[:4]))
+    from torch.overrides import TorchFunctionMode
+
+    class Mode(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        assert not taken()
+    with pytest.raises(AssertionError):
+        fp8_decode_attention(q.contiguous().float(), *caches, lens, tables, 0.1)
+    with pytest.raises(AssertionError):
+        store_fp8_kvcache(k, v[:4], *caches, slots)
+    with pytest.raises(RuntimeError, match="status -2"):
+        varlen_attention(q.contiguous(), k, v, lens[:2].cumsum(0, dtype=torch.int32) - 1,
+                         lens[:2].cumsum(0, dtype=torch.int32) - 1, 1, softmax_scale=-1.0)
