@@ -47,9 +47,10 @@
 //    measured 2x slower).  A sequence that fits in one split is written
 //    directly by the split kernel.
 //  * Grids of many rounds (over 512 eight-wave workgroups) run compacted
-//    work items longest-first: a pre-pass ranks the sequences by length on
-//    the device and lists their valid splits, so short sequences fill the
-//    last round and empty splits exit at the end of the grid.
+//    work items longest-first: a pre-pass on the device lists the valid
+//    splits, full ones first, then the sequences' last ones by length, so
+//    short ones fill the last round and empty splits exit at the end of the
+//    grid.
 //  * Two workgroup shapes, chosen from shapes alone: 8 waves (all 8 kv
 //    heads of a token range, whole 1 KiB token rows, 132 KB of LDS: one per
 //    CU), and 4 waves (half a token row each, two per CU) for grids of many
@@ -105,6 +106,9 @@ struct SplitRule {
   // 1 / the splits that run at once (CUs over workgroups per split, less
   // half a split per sequence), and 1 / splits
   float inv_slots, inv_splits;
+  // with work items, what the pre-pass left: the item count and
+  // split_tokens; else null
+  int* info;
 };
 
 struct DecodeArgs {
@@ -121,9 +125,8 @@ struct DecodeArgs {
   // Work items longest-first (grids of many rounds, else null): item i is
   // (sequence, split, length, block id of the split's first page), for
   // the valid splits of the sequences in order of decreasing length, and
-  // item_count of them are valid.
+  // rule.info[0] of them are valid.
   const int4* items;
-  const int* item_count;
   int batch, hq, hk, group, qgroups, bs, w, splits, pages_per_split;
   SplitRule rule;
   int64_t num_blocks;
@@ -153,6 +156,18 @@ __device__ __forceinline__ int wave_max_u31(int v) {  // of values >= 0
   return max((int)r32[0], (int)r32[1]);
 }
 
+__device__ __forceinline__ int steps_of_length(int len, const SplitRule& r) {
+  return (max(0, min(len, r.max_tokens)) + kStep - 1) / kStep;
+}
+// (longest / splits is at least 1 / longest away from a whole number or on
+// it, 2^-17 with max_tokens <= 2^22, so the float product never rounds it
+// down past one)
+__device__ __forceinline__ int split_tokens_from(int steps, int longest, const SplitRule& r) {
+  const int per = max((int)ceilf(fmaxf((float)steps * r.inv_slots, (float)longest * r.inv_splits)),
+                      kMinSplitSteps);
+  return min(per * kStep, r.fixed);
+}
+
 // The tokens per split of this step, from the lengths on the device: a
 // table as wide as the longest context a graph was captured for says
 // nothing about the lengths, and a wave's chain of 32-token steps (about 2
@@ -161,27 +176,27 @@ __device__ __forceinline__ int wave_max_u31(int v) {  // of values >= 0
 // split per sequence for its ragged end); a split has two steps at least,
 // the longest sequence fits in the splits there are, and the shape's own
 // split, which fills the chip when every sequence is full, is the most.
-// Whole steps, not whole pages.  Measured against the shape's split, us:
+// Whole steps, not whole pages.  With work items the pre-pass applies the
+// rule and leaves its result in rule.info.  Measured against the shape's split, us:
 // batch 16, 64 to 4096 tokens under 128-entry tables 77 -> 23 (the layer's
 // step), 8 x 1000 under 128 entries 53 -> 13, 1 x 512 18.6 -> 11.2, 1 x 4096
 // 19.4 -> 13.2.  Every wave of the split kernel and of the
-// merges computes the same value.  (batch <= 256 and max_tokens <= 2^22
+// merges computes the same value.  (batch <= 4096 and max_tokens <= 2^22
 // where it adapts: the sum of steps stays within an int.)
 // `own` is this lane's length, loaded early so that it shares the round trip
 // of the caller's first reads; `len` is the caller's sequence's.
 __device__ __forceinline__ int lane_length(const int32_t* __restrict__ seqlens,
                                            const SplitRule& r) {
   const int lane = threadIdx.x & 63;
-  return r.adapt && r.batch > 1 && lane < r.batch ? seqlens[lane] : 0;
+  return r.adapt && !r.info && r.batch > 1 && lane < r.batch ? seqlens[lane] : 0;
 }
 __device__ __forceinline__ int split_tokens_of(int own, int len,
                                                const int32_t* __restrict__ seqlens,
                                                const SplitRule& r) {
+  if (r.info) return __builtin_amdgcn_readfirstlane(r.info[1]);
   if (!r.adapt) return r.fixed;
   int steps, longest;
-  auto steps_of = [&](int len) {
-    return (max(0, min(len, r.max_tokens)) + kStep - 1) / kStep;
-  };
+  auto steps_of = [&](int len) { return steps_of_length(len, r); };
   if (r.batch == 1) {
     steps = longest = steps_of(len);
   } else {
@@ -194,12 +209,7 @@ __device__ __forceinline__ int split_tokens_of(int own, int len,
     steps = __builtin_amdgcn_readfirstlane(wave_sum_i32(steps));
     longest = __builtin_amdgcn_readfirstlane(wave_max_u31(longest));
   }
-  // (longest / splits is at least 1 / longest away from a whole number or on
-  // it, 2^-17 with these limits, so the float product never rounds it down
-  // past one)
-  const int per = max((int)ceilf(fmaxf((float)steps * r.inv_slots, (float)longest * r.inv_splits)),
-                      kMinSplitSteps);
-  return min(per * kStep, r.fixed);
+  return split_tokens_from(steps, longest, r);
 }
 
 struct StepLoads {
@@ -459,7 +469,15 @@ __device__ __forceinline__ void write_partial(float* po, float* plse, const f32x
 // (132 KB) or two 4-wave ones (66 KB each) per CU.  (A hint of 3 could not
 // be met and left the 4-wave instance at 200 VGPRs instead of 167, with no
 // difference in time.)
-template <typename T, int W>
+//
+// kItems: grid row (z, y) takes work item z * splits + y: full splits first,
+// then the sequences' last ones by length, so the last round holds the short
+// ones; rows past the last item end at once.  (A grid of one round that
+// claimed its items from a counter was slower: 256 x 64-4096 tokens 138
+// against 124 us.)
+// kFollow: the splits follow the lengths; kFixed: they are the shape's.
+enum DecodeMode { kFixed, kFollow, kItems };
+template <typename T, int W, DecodeMode kMode>
 __global__ __launch_bounds__(64 * W)
 __attribute__((amdgpu_waves_per_eu(2, 8)))
 void decode_fp8_kernel(DecodeArgs a) {
@@ -472,79 +490,84 @@ void decode_fp8_kernel(DecodeArgs a) {
   const int lane = threadIdx.x & 63;
   const int g = lane >> 4, n = lane & 15;
   const int unit = blockIdx.x * W + wave;
-  // The sequence, its length and the split's first block id are read
-  // together, first thing, so the first K/V loads wait for one memory round
-  // trip, not a chain of them (readfirstlane is convergent, so the compiler
-  // cannot sink a read below the branches that use it).  The split's first
-  // page, clamped to the table (splits finer than a page may be more than its
-  // entries), is that of the shape's own split; another one is read below.
-  // With work items, grid row (z, y) takes item z * splits + y: the valid
-  // splits of the longest sequences first, short sequences' in the last
-  // round, and the rows past the last item (empty splits) at the end of the
-  // grid.  Splits that follow the lengths put the empty ones last by taking
-  // z as the split (in between, every 2 us wave of them delays the valid ones
-  // behind: batch 16 x 4096 tokens, half of 32 splits empty, 43 against 29
-  // us); the sequences rotate with it, so that one sequence's splits spread
-  // over the XCDs.
-  const int own = lane_length(a.seqlens, a.rule);
-  int b, split, len_raw, blk_first;
-  if (a.items) {
-    const int item = blockIdx.z * a.splits + blockIdx.y;
-    const int4 e = a.items[item];
-    const int count = __builtin_amdgcn_readfirstlane(*a.item_count);
-    b = __builtin_amdgcn_readfirstlane(e.x);
-    split = __builtin_amdgcn_readfirstlane(e.y);
-    len_raw = __builtin_amdgcn_readfirstlane(e.z);
-    blk_first = __builtin_amdgcn_readfirstlane(e.w);
-    if (item >= count) return;
-    if ((unsigned)b >= (unsigned)a.batch || (unsigned)split >= (unsigned)a.splits) return;
-  } else {
-    split = a.rule.adapt ? blockIdx.z : blockIdx.y;
-    b = a.rule.adapt ? (blockIdx.y + blockIdx.z) % a.batch : blockIdx.z;
-    len_raw = __builtin_amdgcn_readfirstlane(a.seqlens[b]);
-    blk_first = __builtin_amdgcn_readfirstlane(
-        a.bt[(int64_t)b * a.w + min(split * a.pages_per_split, a.w - 1)]);
-  }
-  if (unit >= a.hk * a.qgroups) return;
+  const bool unit_ok = unit < a.hk * a.qgroups;
   const int kvh = unit / a.qgroups;
   const int hig = (unit - kvh * a.qgroups) * 16 + n;  // head within its group
   const bool head_ok = hig < a.group;
   const int qh = kvh * a.group + hig;
-  const int split_tokens = a.items ? a.rule.fixed : split_tokens_of(own, len_raw, a.seqlens, a.rule);
-  const int t_begin = split * split_tokens;
-  // tokens past the block table's width are not addressable: ignore them
-  const int L = min(len_raw, a.w * a.bs);
 
-  if (L <= 0) {
-    if (a.splits == 1 && split == 0 && head_ok) {
-      uint16_t* op = a.out + ((int64_t)b * a.hq + qh) * kHeadDim;
+  // one split of one sequence; blk_first: the block id of its first page
+  auto run = [&](int b, int split, int len_raw, int blk_first, int split_tokens) {
+    const int t_begin = split * split_tokens;
+    // tokens past the block table's width are not addressable: ignore them
+    const int L = min(len_raw, a.w * a.bs);
+    if (L <= 0) {
+      if (a.splits == 1 && split == 0 && head_ok) {
+        uint16_t* op = a.out + ((int64_t)b * a.hq + qh) * kHeadDim;
 #pragma unroll
-      for (int dt = 0; dt < 8; ++dt)
-        *reinterpret_cast<u32x2*>(op + 16 * dt + 4 * g) = u32x2{0u, 0u};
+        for (int dt = 0; dt < 8; ++dt)
+          *reinterpret_cast<u32x2*>(op + 16 * dt + 4 * g) = u32x2{0u, 0u};
+      }
+      return;
     }
-    return;
-  }
-  if (t_begin >= L) return;
-  const int t_end = min(L, t_begin + split_tokens);
-  if (split_tokens != a.rule.fixed)
-    blk_first = __builtin_amdgcn_readfirstlane(a.bt[(int64_t)b * a.w + t_begin / a.bs]);
+    if (t_begin >= L) return;
+    const int t_end = min(L, t_begin + split_tokens);
+    if (kMode == kFollow && split_tokens != a.rule.fixed)
+      blk_first = __builtin_amdgcn_readfirstlane(a.bt[(int64_t)b * a.w + t_begin / a.bs]);
 
-  f32x4 acc[8];
-  float m, l;
-  attend_range<T>(a, b, kvh, qh, head_ok, t_begin, t_end, blk_first, lane, kv_lds_all[wave],
-                  s_lds_all[wave], acc, m, l);
+    f32x4 acc[8];
+    float m, l;
+    attend_range<T>(a, b, kvh, qh, head_ok, t_begin, t_end, blk_first, lane, kv_lds_all[wave],
+                    s_lds_all[wave], acc, m, l);
 
-  // splits that hold tokens of this sequence; a sequence that fits in one
-  // split is written here directly
-  const int nvalid = min(a.splits, (L + split_tokens - 1) / split_tokens);
-  if (!head_ok) return;
-  if (nvalid == 1) {
-    write_output<T>(a.out + ((int64_t)b * a.hq + qh) * kHeadDim, acc, l, g);
-    return;
+    // splits that hold tokens of this sequence; a sequence that fits in one
+    // split is written here directly
+    const int nvalid = min(a.splits, (L + split_tokens - 1) / split_tokens);
+    if (!head_ok) return;
+    if (nvalid == 1) {
+      write_output<T>(a.out + ((int64_t)b * a.hq + qh) * kHeadDim, acc, l, g);
+      return;
+    }
+    // this split's partial, merged by a combine kernel
+    const int64_t row = ((int64_t)b * a.hq + qh) * a.splits + split;
+    write_partial(a.part_o + row * kHeadDim, a.part_lse + row, acc, m, l, g);
+  };
+
+  if constexpr (kMode == kItems) {
+    const int item = blockIdx.z * a.splits + blockIdx.y;
+    const int4 e = a.items[item];
+    const int count = __builtin_amdgcn_readfirstlane(a.rule.info[0]);
+    const int split_tokens = __builtin_amdgcn_readfirstlane(a.rule.info[1]);
+    const int b = __builtin_amdgcn_readfirstlane(e.x);
+    const int split = __builtin_amdgcn_readfirstlane(e.y);
+    const int len_raw = __builtin_amdgcn_readfirstlane(e.z);
+    const int blk_first = __builtin_amdgcn_readfirstlane(e.w);
+    if (item >= count || !unit_ok) return;
+    if ((unsigned)b >= (unsigned)a.batch || (unsigned)split >= (unsigned)a.splits) return;
+    run(b, split, len_raw, blk_first, split_tokens);
+  } else {
+    // The sequence, its length and the split's first block id are read
+    // together, first thing, so the first K/V loads wait for one memory
+    // round trip, not a chain of them (readfirstlane is convergent, so the
+    // compiler cannot sink a read below the branches that use it).  The
+    // split's first page, clamped to the table (splits finer than a page may
+    // be more than its entries), is that of the shape's own split; another
+    // one is read later.  Splits that follow the lengths put the empty ones
+    // last by taking z as the split (in between, every 2 us wave of them
+    // delays the valid ones behind: batch 16 x 4096 tokens, half of 32
+    // splits empty, 43 against 29 us); the sequences rotate with it, so that
+    // one sequence's splits spread over the XCDs.
+    constexpr bool kAdapt = kMode == kFollow;
+    const int own = kAdapt ? lane_length(a.seqlens, a.rule) : 0;
+    const int split = kAdapt ? blockIdx.z : blockIdx.y;
+    const int b = kAdapt ? (blockIdx.y + blockIdx.z) % a.batch : blockIdx.z;
+    const int len_raw = __builtin_amdgcn_readfirstlane(a.seqlens[b]);
+    const int blk_first = __builtin_amdgcn_readfirstlane(
+        a.bt[(int64_t)b * a.w + min(split * a.pages_per_split, a.w - 1)]);
+    if (!unit_ok) return;
+    run(b, split, len_raw, blk_first,
+        kAdapt ? split_tokens_of(own, len_raw, a.seqlens, a.rule) : a.rule.fixed);
   }
-  // this split's partial, merged by a combine kernel
-  const int64_t row = ((int64_t)b * a.hq + qh) * a.splits + split;
-  write_partial(a.part_o + row * kHeadDim, a.part_lse + row, acc, m, l, g);
 }
 
 // A merge state over some splits of one row, held in plain registers: the
@@ -676,21 +699,22 @@ __device__ __forceinline__ void write_merged(uint16_t* op, float den, f32x4 o) {
 // One wave per (b, h) row: lane (j, i) takes d in [4i, 4i + 4) of splits
 // j, j + 2, ..., kLoopK of them per memory round trip (32 splits: the
 // ragged batch's whole row in one), and the two halves merge across lanes.
+// kRule (all merges): the tokens per split may follow the lengths.
 constexpr int kLoopK = 16;
 
-template <typename T>
+template <typename T, bool kRule>
 __global__ __launch_bounds__(64) void decode_combine_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_lse,
     const int32_t* __restrict__ seqlens, uint16_t* __restrict__ out, int hq,
     SplitRule rule) {
   const int splits = rule.splits;
-  const int own = lane_length(seqlens, rule);
+  const int own = kRule ? lane_length(seqlens, rule) : 0;
   const int row = blockIdx.x;  // b * hq + h
   const int b = row / hq;
   const int lane = threadIdx.x;
   const int j = lane >> 5, i = lane & 31;
   const int L = min(seqlens[b], rule.max_tokens);
-  const int split_tokens = split_tokens_of(own, L, seqlens, rule);
+  const int split_tokens = kRule ? split_tokens_of(own, L, seqlens, rule) : rule.fixed;
   const int nvalid = L <= 0 ? 0 : min(splits, (L + split_tokens - 1) / split_tokens);
   if (nvalid == 1) return;
   const float* lse = part_lse + (int64_t)row * splits;
@@ -710,13 +734,13 @@ __global__ __launch_bounds__(64) void decode_combine_kernel(
 // batches), the reads of unused rows cost more than the round trip, so
 // those keep decode_combine_kernel.  M is the largest valid lse value and
 // the weighted sum runs in split order.
-template <typename T, int S>
+template <typename T, int S, bool kRule>
 __global__ __launch_bounds__(64) void decode_combine_small_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_lse,
     const int32_t* __restrict__ seqlens, uint16_t* __restrict__ out, int hq,
     SplitRule rule) {
   const int splits = rule.splits;
-  const int own = lane_length(seqlens, rule);
+  const int own = kRule ? lane_length(seqlens, rule) : 0;
   const int row = blockIdx.x;  // b * hq + h
   const int b = row / hq;
   const int lane = threadIdx.x;
@@ -733,7 +757,7 @@ __global__ __launch_bounds__(64) void decode_combine_small_kernel(
                          : float2{0.0f, 0.0f};
   }
   const int L = min(seqlens[b], rule.max_tokens);
-  const int split_tokens = split_tokens_of(own, L, seqlens, rule);
+  const int split_tokens = kRule ? split_tokens_of(own, L, seqlens, rule) : rule.fixed;
   const int nvalid = L <= 0 ? 0 : min(splits, (L + split_tokens - 1) / split_tokens);
   if (nvalid == 1) return;
   float M = -INFINITY;
@@ -767,13 +791,13 @@ constexpr int kWideWaves = 4;
 constexpr int kWideK = 8;
 constexpr int kWideThreshold = 64;  // splits above this use the wide merge
 
-template <typename T>
+template <typename T, bool kRule>
 __global__ __launch_bounds__(64 * kWideWaves) void decode_combine_wide_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_lse,
     const int32_t* __restrict__ seqlens, uint16_t* __restrict__ out, int hq,
     SplitRule rule) {
   const int splits = rule.splits;
-  const int own = lane_length(seqlens, rule);
+  const int own = kRule ? lane_length(seqlens, rule) : 0;
   __shared__ float s_m[kWideWaves][8], s_den[kWideWaves][8];
   __shared__ __attribute__((aligned(16))) f32x4 s_o[kWideWaves][8];
   const int row = blockIdx.x;  // b * hq + h
@@ -793,7 +817,7 @@ __global__ __launch_bounds__(64 * kWideWaves) void decode_combine_wide_kernel(
   SplitLoads<kWideK> first;
   load_splits(first, lse, po, 8 * wave + j, 8 * kWideWaves, min(splits, kPass));
   const int L = min(seqlens[b], rule.max_tokens);
-  const int split_tokens = split_tokens_of(own, L, seqlens, rule);
+  const int split_tokens = kRule ? split_tokens_of(own, L, seqlens, rule) : rule.fixed;
   const int nvalid = L <= 0 ? 0 : min(splits, (L + split_tokens - 1) / split_tokens);
   if (nvalid == 1) return;  // written by the split kernel
   float m = -INFINITY, den = 0.0f;
@@ -821,52 +845,92 @@ __global__ __launch_bounds__(64 * kWideWaves) void decode_combine_wide_kernel(
   write_merged<T>(out + (int64_t)row * kHeadDim + d, den, o);
 }
 
-// The longest-first work items of a split grid of many rounds: workgroup
-// b ranks sequence b by its length (clamped to the table; ties by index,
-// so the order is total) and sums the valid splits of the sequences ahead
-// of it, which is where its items start; it writes one item per valid
-// split of its own.  Workgroup 0 also writes the item count.  The block
-// ids are read alongside the lengths, so the items cost one memory round
-// trip before the writes.
+// The work items of a split grid of many rounds, the long ones first: every
+// workgroup finds the tokens per split from all the lengths (split_tokens_of's
+// rule); workgroup b counts the full splits of the sequences before b and
+// the partial splits longer than its own (ties by index, so the order is
+// total), which is where its items go, and writes one per valid split.
+// Workgroup 0 also writes rule.info: the item count and the tokens per split.
 constexpr int kOrderThreads = 256;
 constexpr int kOrderMaxBatch = 4096;
 
 __global__ __launch_bounds__(kOrderThreads) void decode_order_kernel(
     const int32_t* __restrict__ seqlens, const int32_t* __restrict__ bt, int4* __restrict__ items,
-    int* __restrict__ item_count, int batch, int w, int max_tokens, int splits,
-    int pages_per_split, int split_tokens) {
-  __shared__ int s_off[kOrderThreads / 64], s_tot[kOrderThreads / 64];
+    int bs, int w, SplitRule rule) {
+  constexpr int kWaves = kOrderThreads / 64;
+  __shared__ int s_steps[kWaves], s_long[kWaves], s_off[kWaves], s_tot[kWaves], s_part[kWaves];
   const int b = blockIdx.x;
   const int tid = threadIdx.x;
   const int len_b = seqlens[b];
-  // this thread's first split's block id, read with the lengths
-  const int blk0 = tid < splits ? bt[(int64_t)b * w + tid * pages_per_split] : 0;
-  const int key = max(0, min(len_b, max_tokens));
-  const int nv_b = min(splits, (key + split_tokens - 1) / split_tokens);
-  int off = 0, tot = 0;
-  for (int j = tid; j < batch; j += kOrderThreads) {
-    const int kj = max(0, min(seqlens[j], max_tokens));
-    const int nj = min(splits, (kj + split_tokens - 1) / split_tokens);
-    off += (kj > key || (kj == key && j < b)) ? nj : 0;
-    tot += nj;
+  // this thread's first split's block id under the shape's own split, read
+  // with the lengths
+  const int fixed_page = tid * (rule.fixed / bs);
+  const int blk_fixed = tid < rule.splits && fixed_page < w ? bt[(int64_t)b * w + fixed_page] : 0;
+  int split_tokens = rule.fixed;
+  if (rule.adapt) {
+    int steps = 0, longest = 0;
+    for (int j = tid; j < rule.batch; j += kOrderThreads) {
+      const int n = steps_of_length(seqlens[j], rule);
+      steps += n;
+      longest = max(longest, n);
+    }
+    steps = wave_sum_i32(steps);
+    longest = wave_max_u31(longest);
+    if ((tid & 63) == 0) {
+      s_steps[tid >> 6] = steps;
+      s_long[tid >> 6] = longest;
+    }
+    __syncthreads();
+    steps = longest = 0;
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) {
+      steps += s_steps[i];
+      longest = max(longest, s_long[i]);
+    }
+    split_tokens = split_tokens_from(steps, longest, rule);
   }
+  // A sequence's full splits come in the order of its index, ahead of every
+  // partial split; its partial one, if any, by the tokens in it (ties by
+  // index).
+  const int key = max(0, min(len_b, rule.max_tokens));
+  const int full_b = key / split_tokens;
+  const int rest_b = key - full_b * split_tokens;
+  int off = 0, tot = 0, ahead = 0, parts = 0;
+  for (int j = tid; j < rule.batch; j += kOrderThreads) {
+    const int kj = max(0, min(seqlens[j], rule.max_tokens));
+    const int full = kj / split_tokens, rest = kj - full * split_tokens;
+    off += j < b ? full : 0;
+    tot += full;
+    ahead += rest > rest_b || (rest == rest_b && j < b) ? rest > 0 : 0;
+    parts += rest > 0;
+  }
+  // (both at most 2^12 sequences: one sum)
+  ahead = wave_sum_i32(ahead | parts << 16);
   off = wave_sum_i32(off);
   tot = wave_sum_i32(tot);
   if ((tid & 63) == 0) {
     s_off[tid >> 6] = off;
     s_tot[tid >> 6] = tot;
+    s_part[tid >> 6] = ahead;
   }
   __syncthreads();
-  int first = 0, count = 0;
+  int first = 0, fulls = 0, part = 0;
 #pragma unroll
-  for (int i = 0; i < kOrderThreads / 64; ++i) {
+  for (int i = 0; i < kWaves; ++i) {
     first += s_off[i];
-    count += s_tot[i];
+    fulls += s_tot[i];
+    part += s_part[i];
   }
-  if (b == 0 && tid == 0) *item_count = count;
-  if (tid < nv_b) items[first + tid] = int4{b, tid, len_b, blk0};
-  for (int sp = tid + kOrderThreads; sp < nv_b; sp += kOrderThreads)
-    items[first + sp] = int4{b, sp, len_b, bt[(int64_t)b * w + sp * pages_per_split]};
+  const int count = fulls + (part >> 16);
+  if (b == 0 && tid < 2) rule.info[tid] = tid == 0 ? count : split_tokens;
+  const int nv_b = full_b + (rest_b > 0);
+  for (int sp = tid; sp < nv_b; sp += kOrderThreads) {
+    // (a split with tokens starts inside the table)
+    const int blk = sp == tid && split_tokens == rule.fixed
+                        ? blk_fixed
+                        : bt[(int64_t)b * w + (int64_t)sp * split_tokens / bs];
+    items[sp < full_b ? first + sp : fulls + (part & 0xFFFF)] = int4{b, sp, len_b, blk};
+  }
 }
 
 // units of up to 16 q heads per kv head: a group above 16 that is not a
@@ -906,42 +970,56 @@ static hipError_t launch_decode(const DecodeArgs& a, int batch, hipStream_t stre
   const int units = a.hk * a.qgroups;
   const int64_t wide_wgs = (int64_t)((units + kWavesPerWG - 1) / kWavesPerWG) * a.splits * batch;
   if (a.items) {
+    // 8-wave workgroups also run the work items when every wave has a unit:
+    // with the short sequences last, their longer units no longer lengthen
+    // the tail (ragged batch 256: 425-426 against 433-435 us with 4 waves).
+    const bool wide = units >= kWavesPerWG;
+    const int per_wg = wide ? kWavesPerWG : kNarrowWaves;
+    const dim3 grid((unsigned)((units + per_wg - 1) / per_wg), (unsigned)a.splits,
+                    (unsigned)batch);
     hipLaunchKernelGGL(decode_order_kernel, dim3((unsigned)batch), dim3(kOrderThreads), 0, stream,
-                       a.seqlens, a.bt, const_cast<int4*>(a.items),
-                       const_cast<int*>(a.item_count), batch, a.w, a.w * a.bs, a.splits,
-                       a.pages_per_split, a.pages_per_split * a.bs);
+                       a.seqlens, a.bt, const_cast<int4*>(a.items), a.bs, a.w, a.rule);
     const hipError_t eo = hipGetLastError();
     if (eo != hipSuccess) return eo;
-  }
-  // 8-wave workgroups also run the work items when every wave has a unit:
-  // with the short sequences last, their longer units no longer lengthen
-  // the tail (ragged batch 256: 425-426 against 433-435 us with 4 waves)
-  if (wide_wgs <= kWideGridMax || (a.items && units >= kWavesPerWG)) {
+    if (wide)
+      hipLaunchKernelGGL((decode_fp8_kernel<T, kWavesPerWG, kItems>), grid, dim3(64 * kWavesPerWG),
+                         0, stream, a);
+    else
+      hipLaunchKernelGGL((decode_fp8_kernel<T, kNarrowWaves, kItems>), grid,
+                         dim3(64 * kNarrowWaves), 0, stream, a);
+  } else if (wide_wgs <= kWideGridMax) {
     dim3 grid((unsigned)((units + kWavesPerWG - 1) / kWavesPerWG), (unsigned)a.splits,
               (unsigned)batch);
-    if (a.rule.adapt) std::swap(grid.y, grid.z);
-    hipLaunchKernelGGL((decode_fp8_kernel<T, kWavesPerWG>), grid, dim3(64 * kWavesPerWG), 0,
-                       stream, a);
+    if (a.rule.adapt) {
+      std::swap(grid.y, grid.z);
+      hipLaunchKernelGGL((decode_fp8_kernel<T, kWavesPerWG, kFollow>), grid,
+                         dim3(64 * kWavesPerWG), 0, stream, a);
+    } else {
+      hipLaunchKernelGGL((decode_fp8_kernel<T, kWavesPerWG, kFixed>), grid,
+                         dim3(64 * kWavesPerWG), 0, stream, a);
+    }
   } else {
     const dim3 grid((unsigned)((units + kNarrowWaves - 1) / kNarrowWaves), (unsigned)a.splits,
                     (unsigned)batch);
-    hipLaunchKernelGGL((decode_fp8_kernel<T, kNarrowWaves>), grid, dim3(64 * kNarrowWaves), 0,
-                       stream, a);
+    hipLaunchKernelGGL((decode_fp8_kernel<T, kNarrowWaves, kFixed>), grid,
+                       dim3(64 * kNarrowWaves), 0, stream, a);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || a.splits == 1) return e;
+  const bool rule = a.rule.adapt || a.rule.info;
+  auto merge = [&](auto kernel, dim3 grid, unsigned threads) {
+    hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, stream, a.part_o, a.part_lse, a.seqlens,
+                       a.out, a.hq, a.rule);
+  };
+  const unsigned rows = (unsigned)(batch * a.hq);
   if (a.splits > kWideThreshold)
-    hipLaunchKernelGGL(decode_combine_wide_kernel<T>, dim3((unsigned)(batch * a.hq), 4u),
-                       dim3(64 * kWideWaves), 0, stream, a.part_o, a.part_lse, a.seqlens, a.out,
-                       a.hq, a.rule);
+    merge(rule ? decode_combine_wide_kernel<T, true> : decode_combine_wide_kernel<T, false>,
+          dim3(rows, 4u), 64 * kWideWaves);
   else if (a.splits <= 8)
-    hipLaunchKernelGGL((decode_combine_small_kernel<T, 8>), dim3((unsigned)(batch * a.hq)),
-                       dim3(64), 0, stream, a.part_o, a.part_lse, a.seqlens, a.out, a.hq,
-                       a.rule);
+    merge(rule ? decode_combine_small_kernel<T, 8, true> : decode_combine_small_kernel<T, 8, false>,
+          dim3(rows), 64);
   else
-    hipLaunchKernelGGL(decode_combine_kernel<T>, dim3((unsigned)(batch * a.hq)), dim3(64), 0,
-                       stream, a.part_o, a.part_lse, a.seqlens, a.out, a.hq,
-                       a.rule);
+    merge(rule ? decode_combine_kernel<T, true> : decode_combine_kernel<T, false>, dim3(rows), 64);
   return hipGetLastError();
 }
 
@@ -1040,13 +1118,13 @@ static int decode_checked(const void* query, const void* k_cache, const void* v_
   a.part_o = need > 0 ? (float*)workspace : nullptr;
   a.part_lse = need > 0 ? a.part_o + (size_t)batch * num_q_heads * num_splits * head_dim
                         : nullptr;
-  // the work items follow the partials: a 16-byte slot for the count, then
-  // one 16-byte item per (sequence, split)
+  // the work items follow the partials: a 16-byte slot for the pre-pass's
+  // results (SplitRule::info), then one 16-byte item per (sequence, split)
   a.items = nullptr;
-  a.item_count = nullptr;
+  int* info = nullptr;
   if (need > 0 && ordered_of(batch, num_kv_heads, qgroups_of(group), num_splits)) {
     uint8_t* base = (uint8_t*)workspace + partials_bytes(batch, num_q_heads, num_splits);
-    a.item_count = (const int*)base;
+    info = (int*)base;
     a.items = (const int4*)(base + sizeof(int4));
   }
   a.batch = batch;
@@ -1058,8 +1136,9 @@ static int decode_checked(const void* query, const void* k_cache, const void* v_
   a.w = max_blocks_per_seq;
   a.splits = num_splits;
   a.pages_per_split = pages_per_split_of(num_splits, max_blocks_per_seq);
-  // Splits follow the lengths on the device where the grid is at most about
-  // two rounds of 8-wave workgroups, one per CU
+  // Splits follow the lengths on the device, in the pre-pass where there is
+  // one, else in the kernels where the grid is at most about two rounds of
+  // 8-wave workgroups, one per CU
   const int64_t per_split = (num_kv_heads * a.qgroups + kWavesPerWG - 1) / kWavesPerWG;
   const int64_t slots =
       std::max<int64_t>(256 / per_split - batch / 2, std::max<int64_t>(128 / per_split, 1));
@@ -1067,12 +1146,13 @@ static int decode_checked(const void* query, const void* k_cache, const void* v_
   // the shapes whose tables fit the lengths: 64 x 4096 tokens would pay 0.5
   // us for the same splits.)
   const bool fine = num_splits > max_blocks_per_seq;
-  const bool adapt = (fine || (a.pages_per_split > 1 && num_splits > 8)) && !a.items &&
-                     batch <= 256 && per_split * num_splits * batch <= kWideGridMax &&
+  const bool adapt = (fine || (a.pages_per_split > 1 && num_splits > 8)) &&
+                     (a.items || (batch <= 256 &&
+                                  per_split * num_splits * batch <= kWideGridMax)) &&
                      (int64_t)max_blocks_per_seq * block_size <= 1 << 22;
   a.rule = SplitRule{batch, num_splits, a.pages_per_split * block_size,
                      max_blocks_per_seq * block_size, adapt, 1.0f / (float)slots,
-                     1.0f / (float)num_splits};
+                     1.0f / (float)num_splits, info};
   a.num_blocks = num_blocks;
   a.scale_log2 = softmax_scale * kLog2e;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);

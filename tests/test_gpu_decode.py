@@ -575,3 +575,23 @@ def test_decode_splits_follow_the_lengths_of_each_replay():
         eager = fp8_decode_attention(q, *caches, static.clone(), tables, 0.088)
         torch.cuda.synchronize()
         assert torch.equal(out, eager), now
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lens,width", [
+    # no full split, only full splits, ties, empty sequences; splits that
+    # follow the lengths under tables of 128 entries (32 splits, 40 sequences)
+    ([1 + i % 3 for i in range(40)], 128),
+    ([0] * 39 + [9000], 128), ([1024] * 20 + [0] * 5 + [2048, 4096] * 8, 128),
+    ([64 * (1 + i % 7) + i % 2 for i in range(40)], 128),
+    # tables that fit (16 splits): the shape's own split
+    ([4 * 256 * (1 + i % 16) - i % 5 for i in range(40)], 64),
+])
+def test_decode_work_items_full_splits_then_the_rest(lens, width, dtype):
+    nb = sum((n + H.BLOCK - 1) // H.BLOCK for n in lens) + 2
+    query, tables, caches = _setup(661 + len(lens), lens, 32, 8, nb, dtype)
+    if width > tables.shape[1]:
+        tables = torch.nn.functional.pad(tables, (0, width - tables.shape[1]), value=-1)
+    assert len(lens) * decode_num_splits(len(lens), 32, 8, width, H.BLOCK) > 512
+    _, out = _run_and_check(query, lens, tables, caches)
+    assert all(torch.all(out[i].float() == 0) for i, n in enumerate(lens) if n == 0)
