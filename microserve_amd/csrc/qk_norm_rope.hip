@@ -27,8 +27,8 @@
 //   Store: the bytes and scales of store_fp8_kvcache on the rotated k and on
 //   v (microserve/layers/fp8_kv_cache.py:11-39).
 //
-// Work layout: eight lanes own a chunk of up to four rows of one kind (q, k
-// or v heads) of one token; lane l holds elements [8l, 8l+8) and
+// Work layout: eight lanes own a chunk of up to four rows (one in a small
+// grid, see kNrSmallBlocks) of one kind (q, k or v heads) of one token; lane l holds elements [8l, 8l+8) and
 // [64+8l, 64+8l+8) of each, so rotate_half's pairs (d, d+64) meet in one
 // lane and the only cross-lane traffic is the two DPP reductions.  The
 // token's rotary rows and the norm weights are unpacked once per chunk, not
@@ -45,7 +45,6 @@ namespace mskv {
 
 constexpr int kNrThreads = 256;
 constexpr int kNrGroups = kNrThreads / 8;  // 8-lane groups per workgroup
-constexpr int kNrChunk = 4;                // rows per group: heads of one kind, one token
 
 struct NormRopeArgs {
   const uint16_t* q;
@@ -238,7 +237,7 @@ __device__ __forceinline__ void norm_rope_row_f16(const NormRopeArgs& a, bool ha
 // Each 8-lane group owns one chunk: up to kNrChunk consecutive heads of one
 // kind of one token.  It issues the loads of all its rows first, then
 // unpacks the token's rotary values and the norm weights once for them.
-template <typename T, typename SlotT>
+template <typename T, typename SlotT, int kNrChunk>
 __global__ __launch_bounds__(kNrThreads) void qk_norm_rope_store_kernel(NormRopeArgs a) {
   const int sub = threadIdx.x & 7;
   const int64_t chunk = (int64_t)blockIdx.x * kNrGroups + (threadIdx.x >> 3);
@@ -370,16 +369,38 @@ __global__ __launch_bounds__(kNrThreads) void qk_norm_rope_store_kernel(NormRope
   }
 }
 
-template <typename T>
-static hipError_t launch_norm_rope(const NormRopeArgs& a, int slot_dtype, hipStream_t stream) {
+// Up to this many workgroups of single rows, a group takes one row, not four:
+// the grid is too small for VALU issue to bind, and the chain of four rows
+// in a lane sets the time.  Four rows against one (bf16, 32 q / 8 kv heads,
+// us): 16 tokens 8.7 / 6.2, 256 9.1 / 6.5, 1000 12.0 / 9.3 (1500 workgroups),
+// 2000 14.8 / 14.6 (3000), 4000 24.0 / 25.1; 64 q heads, fp16, 1000 tokens
+// 13.8 / 12.5 (2500).  A row's arithmetic is the same in both.
+constexpr int64_t kNrSmallBlocks = 2560;
+
+template <typename T, int kNrChunk>
+static hipError_t launch_chunks(NormRopeArgs a, int64_t num_tokens, int slot_dtype,
+                                hipStream_t stream) {
+  a.cq = (a.hq + kNrChunk - 1) / kNrChunk;
+  a.ck = (a.hk + kNrChunk - 1) / kNrChunk;
+  a.q_chunks = num_tokens * a.cq;
+  a.k_chunks = num_tokens * a.ck;
+  a.chunks = a.q_chunks + 2 * a.k_chunks;
   const int64_t blocks = (a.chunks + kNrGroups - 1) / kNrGroups;
   if (slot_dtype == MSKV_INT64)
-    hipLaunchKernelGGL((qk_norm_rope_store_kernel<T, int64_t>), dim3((unsigned)blocks),
+    hipLaunchKernelGGL((qk_norm_rope_store_kernel<T, int64_t, kNrChunk>), dim3((unsigned)blocks),
                        dim3(kNrThreads), 0, stream, a);
   else
-    hipLaunchKernelGGL((qk_norm_rope_store_kernel<T, int32_t>), dim3((unsigned)blocks),
+    hipLaunchKernelGGL((qk_norm_rope_store_kernel<T, int32_t, kNrChunk>), dim3((unsigned)blocks),
                        dim3(kNrThreads), 0, stream, a);
   return hipGetLastError();
+}
+
+template <typename T>
+static hipError_t launch_norm_rope(const NormRopeArgs& a, int64_t num_tokens, int slot_dtype,
+                                   hipStream_t stream) {
+  return a.rows <= kNrSmallBlocks * kNrGroups
+             ? launch_chunks<T, 1>(a, num_tokens, slot_dtype, stream)
+             : launch_chunks<T, 4>(a, num_tokens, slot_dtype, stream);
 }
 
 }  // namespace mskv
@@ -425,13 +446,8 @@ extern "C" int mskv_qk_norm_rope_store(
                        (uint16_t*)q_out, (uint16_t*)k_out, (uint8_t*)k_cache,
                        (uint8_t*)v_cache, k_scale_cache, v_scale_cache, slot_mapping, rows,
                        num_slots, max_position, num_q_heads, num_kv_heads, heads, eps};
-  a.cq = (num_q_heads + mskv::kNrChunk - 1) / mskv::kNrChunk;
-  a.ck = (num_kv_heads + mskv::kNrChunk - 1) / mskv::kNrChunk;
-  a.q_chunks = num_tokens * a.cq;
-  a.k_chunks = num_tokens * a.ck;
-  a.chunks = a.q_chunks + 2 * a.k_chunks;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const hipError_t e = act_dtype == MSKV_BFLOAT16 ? mskv::launch_norm_rope<__bf16>(a, slot_dtype, s)
-                                                   : mskv::launch_norm_rope<_Float16>(a, slot_dtype, s);
+  const hipError_t e = act_dtype == MSKV_BFLOAT16 ? mskv::launch_norm_rope<__bf16>(a, num_tokens, slot_dtype, s)
+                                                   : mskv::launch_norm_rope<_Float16>(a, num_tokens, slot_dtype, s);
   return (int)e;
 }

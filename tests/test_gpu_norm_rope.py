@@ -240,3 +240,33 @@ def test_attention_forward_fused_equals_unfused(mode):
     assert torch.equal(outs[0], outs[1])
     for a, b in zip(*caches):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hk", [(32, 8), (5, 3)])
+def test_one_row_and_four_row_chunks_agree(hq, hk, dtype):
+    """A call past the small grid's limit (2560 workgroups of 32 rows) takes
+    four rows per lane group; the same tokens in two calls below it take one.
+    Outputs, cache bytes and scales are the same bits, head counts that are
+    not multiples of four included."""
+    from tests import gpu_helpers as H
+    n = 2560 * 32 // (hq + 2 * hk) + 1
+    gen = torch.Generator(device=H.DEV).manual_seed(911)
+    qkv = torch.randn(n, (hq + 2 * hk) * H.D, generator=gen, device=H.DEV).to(dtype)
+    q, k, v = (t.view(n, -1, H.D) for t in
+               qkv.split((hq * H.D, hk * H.D, hk * H.D), -1))
+    w = torch.randn(H.D, generator=gen, device=H.DEV).to(dtype)
+    cos, sin = (torch.randn(64, H.D, generator=gen, device=H.DEV).to(dtype) for _ in range(2))
+    pos = torch.arange(n, device=H.DEV) % 65          # position 64 is past the tables
+    blocks = (n + H.BLOCK - 1) // H.BLOCK
+    slots = torch.randperm(blocks * H.BLOCK, generator=gen, device=H.DEV)[:n]
+    whole, parts = H.alloc_cache(blocks, H.BLOCK, hk), H.alloc_cache(blocks, H.BLOCK, hk)
+    got = qk_norm_rope_store(pos, q, k, v, w, w, 1e-6, cos, sin, *whole, slots)
+    halves = [qk_norm_rope_store(pos[s], q[s], k[s], v[s], w, w, 1e-6, cos, sin, *parts, slots[s])
+              for s in (slice(0, n // 2), slice(n // 2, n))]
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert torch.equal(got[i], torch.cat([h[i] for h in halves]))
+    for a, b in zip(whole, parts):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
