@@ -9,21 +9,30 @@ silently take another path.
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
 
 import torch  # noqa: F401  (the extension below uses its libraries)
 
-try:
-    from microserve_amd import _fast_calls as fast
-except ImportError as e:  # raised on use: the package must import to be built
-    class _NotBuilt:
-        why = e
 
-        def __getattr__(self, name):
-            raise RuntimeError("microserve_amd._fast_calls is not built: run "
-                               f"`python -m microserve_amd.build` ({self.why})")
+class _NotBuilt:
+    """Stands in for the native call paths until they are built (the package
+    must import to be built): raises on use."""
 
-    fast = _NotBuilt()
+    def __getattr__(self, name):
+        raise RuntimeError("microserve_amd._fast_calls is not built: run "
+                           "`python -m microserve_amd.build`")
+
+
+def _import_fast():
+    importlib.invalidate_caches()
+    try:
+        return importlib.import_module("microserve_amd._fast_calls")
+    except ImportError:
+        return _NotBuilt()
+
+
+fast = _import_fast()
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libmskv.so")
@@ -89,7 +98,7 @@ _lib = None
 
 def load() -> ctypes.CDLL:
     """Load libmskv.so once; raise with a build hint if it is absent."""
-    global _lib
+    global _lib, fast
     if _lib is not None:
         return _lib
     if not os.path.exists(LIB_PATH):
@@ -101,6 +110,8 @@ def load() -> ctypes.CDLL:
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
+    if isinstance(fast, _NotBuilt):  # built since this module was imported
+        fast = _import_fast()
     fast.bind({name: ctypes.cast(getattr(lib, name), _vp).value for name in _PROTOS})
     _lib = lib
     return lib
