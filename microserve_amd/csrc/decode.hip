@@ -81,6 +81,9 @@ constexpr int kTargetWaves = 2048;
 // workgroup streams whole contiguous token rows; the waves never synchronize
 // with each other.
 constexpr int kWavesPerWG = 8;
+// Widest table (tokens) whose splits follow the lengths: the sums of steps
+// and the float arithmetic of split_tokens_from hold up to it
+constexpr int64_t kFollowMaxTokens = 1 << 22;
 // Largest split partials that splits finer than a page may ask for
 constexpr int64_t kFinePartialBytes = 16 << 20;
 constexpr int kNarrowWaves = 4;       // workgroup shape for grids of many rounds
@@ -1044,8 +1047,12 @@ extern "C" int mskv_decode_num_splits(int batch, int num_q_heads,
   int64_t splits = (w + pps - 1) / pps;
   // A page per split leaves half the waves idle: finer splits, of two steps at least,
   // up to two per wave slot (one is expected to run, see split_tokens_of),
-  // as long as the grid and the partials stay small
-  if (splits > 1 && 2 * w * base <= mskv::kTargetWaves && block_size > 0) {
+  // as long as the grid and the partials stay small.  Only where they follow
+  // the lengths: at the shape's own split a page each, more splits than
+  // table entries would start past an int's tokens at the largest pages
+  // (512 splits of 2^23 tokens).
+  if (splits > 1 && 2 * w * base <= mskv::kTargetWaves && block_size > 0 &&
+      (int64_t)w * block_size <= mskv::kFollowMaxTokens) {
     const int64_t per = (base / batch + mskv::kWavesPerWG - 1) / mskv::kWavesPerWG * batch;
     int64_t fine = 2 * mskv::kTargetWaves / base;
     fine = std::min(fine, (int64_t)w * block_size / (mskv::kMinSplitSteps * mskv::kStep));
@@ -1149,7 +1156,7 @@ static int decode_checked(const void* query, const void* k_cache, const void* v_
   const bool adapt = (fine || (a.pages_per_split > 1 && num_splits > 8)) &&
                      (a.items || (batch <= 256 &&
                                   per_split * num_splits * batch <= kWideGridMax)) &&
-                     (int64_t)max_blocks_per_seq * block_size <= 1 << 22;
+                     (int64_t)max_blocks_per_seq * block_size <= kFollowMaxTokens;
   a.rule = SplitRule{batch, num_splits, a.pages_per_split * block_size,
                      max_blocks_per_seq * block_size, adapt, 1.0f / (float)slots,
                      1.0f / (float)num_splits, info};

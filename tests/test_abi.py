@@ -58,6 +58,24 @@ def test_split_policy_depends_on_shapes_only():
     assert lib.mskv_decode_workspace_bytes(256, 32, 8, 128, 31) == part + 16 + 256 * 31 * 16
 
 
+def test_every_split_starts_within_an_int_of_tokens():
+    """A split's first token is split * (pages per split) * block_size in 32
+    bits; pages may hold millions of tokens, and a page's splits finer than
+    itself must not multiply past that."""
+    lib = _lib.load()
+    for batch in (1, 2, 16, 300):
+        for hq, hk in ((8, 1), (32, 8), (16, 16)):
+            for w in (1, 2, 3, 64, 1000):
+                for block in (32, 256, 1 << 12, 1 << 20, 1 << 22, 1 << 23, (1 << 24) - 32):
+                    if block * hk * 128 > 0x7FFFFFFF or w * block >= 1 << 30:
+                        continue  # rejected by the call itself
+                    s = lib.mskv_decode_num_splits(batch, hq, hk, w, block)
+                    pages = -(-w // s)
+                    assert (s - 1) * pages * block <= 0x7FFFFFFF, (batch, hq, hk, w, block, s)
+                    # more splits than pages only where they follow the lengths
+                    assert s <= w or w * block <= 1 << 22, (batch, hq, hk, w, block, s)
+
+
 def test_argument_validation_without_launch():
     lib = _lib.load()
     EINVAL, EUNSUP, EWS = -1, -2, -3
