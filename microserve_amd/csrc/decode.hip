@@ -458,14 +458,17 @@ __device__ __forceinline__ void write_output(uint16_t* op, const f32x4 (&acc)[8]
   }
 }
 
-// a split's partial: o / l and m + log2 l (-inf when it saw no token)
+// a split's partial: o / l and m + log2 l (-inf when it saw no token).  A NaN
+// l (a NaN query, key or scale) is left as +inf: every merge weighs it with
+// 2^(inf - inf), so the row comes out NaN, as it does from a single split,
+// and is not taken for a split without tokens.
 __device__ __forceinline__ void write_partial(float* po, float* plse, const f32x4 (&acc)[8],
                                               float m, float l, int g) {
   const float inv = l > 0.0f ? 1.0f / l : 0.0f;
 #pragma unroll
   for (int dt = 0; dt < 8; ++dt)
     *reinterpret_cast<f32x4*>(po + 16 * dt + 4 * g) = acc[dt] * inv;
-  if (g == 0) *plse = l > 0.0f ? m + __log2f(l) : -INFINITY;
+  if (g == 0) *plse = is_nan(l) ? INFINITY : l > 0.0f ? m + __log2f(l) : -INFINITY;
 }
 
 // 2 waves per SIMD, the occupancy the LDS allows: one 8-wave workgroup

@@ -173,6 +173,12 @@ __device__ __forceinline__ float exp2_fast(float x) {
   return __builtin_amdgcn_exp2f(x);
 }
 
+// Tested on the bits: -fno-honor-nans lets the compiler assume that no
+// floating-point comparison sees a NaN.
+__device__ __forceinline__ bool is_nan(float x) {
+  return (__float_as_uint(x) & 0x7FFFFFFFu) > 0x7F800000u;
+}
+
 __device__ __forceinline__ float wave_max_xor(float v, int mask) {
   return fmaxf(v, __shfl_xor(v, mask));
 }

@@ -577,9 +577,14 @@ __global__ __launch_bounds__(PShape::threads, 2) void prefill_fp8_kernel(Prefill
     const int qhb = kvh * group + qgi * 16 + n_out - nq * gc;
     const int64_t row = (int64_t)(q_begin + qi) * hq + qhb;
     if constexpr (kSplit) {
+      // (with a NaN denominator the partial is NaN: it gets the largest
+      // weight, so the merged row is NaN, as the unsplit kernel's is, and
+      // the range is not taken for an empty one)
       if (g == 0)
-        part_lse[row * splits + max(split, 0)] =
-            split < 0 ? kPWritten : lt > 0.0f ? m[b] + __log2f(lt) : -INFINITY;
+        part_lse[row * splits + max(split, 0)] = split < 0      ? kPWritten
+                                                 : is_nan(lt)   ? FLT_MAX
+                                                 : lt > 0.0f    ? m[b] + __log2f(lt)
+                                                                : -INFINITY;
       if (split >= 0) {
         float* po = part_o + (row * splits + split) * kHeadDim;
 #pragma unroll

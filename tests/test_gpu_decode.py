@@ -595,3 +595,33 @@ def test_decode_work_items_full_splits_then_the_rest(lens, width, dtype):
     assert len(lens) * decode_num_splits(len(lens), 32, 8, width, H.BLOCK) > 512
     _, out = _run_and_check(query, lens, tables, caches)
     assert all(torch.all(out[i].float() == 0) for i, n in enumerate(lens) if n == 0)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hk,lens,width", [
+    (32, 8, [300, 200], 2),            # splits finer than a page, the small merge or the loop
+    (32, 8, [3000, 900, 40], 64),      # splits that follow the lengths
+    (16, 8, [2000], 0), (64, 8, [9000], 0),          # one sequence: few splits, the wide merge
+    (32, 8, [700 + i for i in range(40)], 128),      # work items
+    (32, 8, [1000] * 64, 0),                         # the shape's own splits
+])
+def test_decode_keeps_a_nan_row_in_every_layout(hq, hk, lens, width, dtype):
+    """A NaN query row, and the rows of a sequence with a NaN key scale at its
+    last token, are NaN and every other row is finite, however the tokens
+    are split and merged."""
+    nb = sum((n + H.BLOCK - 1) // H.BLOCK for n in lens) + 2
+    query, tables, caches = _setup(671 + len(lens), lens, hq, hk, nb, dtype)
+    if width > tables.shape[1]:
+        tables = torch.nn.functional.pad(tables, (0, width - tables.shape[1]), value=-1)
+    query[0, 1] = float("nan")
+    last, n = len(lens) - 1, lens[-1]
+    want = torch.zeros(query.shape, dtype=torch.bool)
+    want[0, 1] = True
+    block = int(tables[last, (n - 1) // H.BLOCK])
+    caches[2][block, (n - 1) % H.BLOCK, hk - 1] = float("nan")
+    want[last, (hk - 1) * (hq // hk):] = True
+    out = fp8_decode_attention(query.to(H.DEV), *caches,
+                               torch.tensor(lens, dtype=torch.int32, device=H.DEV),
+                               tables.to(H.DEV), 0.088)
+    torch.cuda.synchronize()
+    assert torch.equal(torch.isnan(out.float().cpu()), want)

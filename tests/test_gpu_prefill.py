@@ -303,3 +303,19 @@ def test_prefill_split_under_capture_replays_the_eager_result():
         again = fp8_chunk_prefill_attention(q, *caches, t, 3000, 0.088)
         torch.cuda.synchronize()
         assert torch.equal(out, eager) and torch.equal(again, eager)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("at", [0, 700, 2999, 3040])
+def test_prefill_split_keeps_a_nan_key(at, dtype):
+    """A NaN key scale (a NaN that was stored) makes every row that sees the
+    key NaN and no other, whichever range of the keys holds it."""
+    new, cached = 64, 3000
+    query, tables, caches, cu_q, cu_k = _varlen_setup(301, [new], [new + cached], 32, 8, dtype)
+    block = int(tables[0, at // H.BLOCK])
+    caches[2][block, at % H.BLOCK] = float("nan")
+    out = fp8_chunk_prefill_attention(query.to(H.DEV), *caches, tables.to(H.DEV), cached, 0.088)
+    torch.cuda.synchronize()
+    sees = cached + torch.arange(new) >= at
+    nan = torch.isnan(out.float().cpu())
+    assert torch.equal(nan.all(-1).all(-1), sees) and torch.equal(nan.any(-1).any(-1), sees)
