@@ -699,13 +699,16 @@ static hipError_t launch_prefill(const PrefillArgs& a, int num_seqs, int64_t qbl
 // store, us): 512/7680 210 -> 106, 128/7680 195 -> 53, 64/2000 66 -> 31,
 // 512/1000 54 -> 46, 256/600 39 -> 35; split all the same, 4 x 74/129 went
 // 12.5 -> 18.0 and 509/200 at 64 q heads 33.8 -> 35.8.
-static int prefill_splits(int num_seqs, int64_t max_seqlen_q, int num_q_heads, int num_kv_heads,
-                          int block_size, int max_blocks_per_seq) {
+// The partials hold every row of the query tensor: one with more rows than
+// the grid covers (a padded one, its max_seqlen_q that of the real tokens)
+// is not split, so that they stay below 512 workgroups' rows.
+static int prefill_splits(int num_seqs, int64_t total_q, int64_t max_seqlen_q, int num_q_heads,
+                          int num_kv_heads, int block_size, int max_blocks_per_seq) {
   const int group = num_q_heads / num_kv_heads;
   const int per_wg = 8 * (group < 16 ? 16 / group : 1);
   const int64_t qblocks = (max_seqlen_q + per_wg - 1) / per_wg;
   const int64_t wgs = num_seqs * qblocks * num_kv_heads * ((group + 15) / 16);
-  if (wgs <= 0) return 1;
+  if (wgs <= 0 || wgs > 512 || total_q * num_q_heads > wgs * 8 * 16) return 1;
   const int64_t tiles = (int64_t)max_blocks_per_seq * block_size / kPStep;
   const int64_t most =
       min(min((int64_t)512 / wgs, tiles / kPMinSplitTiles), (int64_t)kPMaxSplits);
@@ -732,7 +735,7 @@ extern "C" size_t mskv_fp8_prefill_workspace_bytes(int num_seqs, int64_t total_q
       num_kv_heads <= 0 || num_q_heads % num_kv_heads != 0 || head_dim != mskv::kHeadDim ||
       block_size <= 0 || block_size % mskv::kPStep != 0 || max_blocks_per_seq <= 0)
     return 0;
-  const int s = mskv::prefill_splits(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads,
+  const int s = mskv::prefill_splits(num_seqs, total_q, max_seqlen_q, num_q_heads, num_kv_heads,
                                      block_size, max_blocks_per_seq);
   return s < 2 ? 0 : (size_t)total_q * num_q_heads * s * (mskv::kHeadDim + 1) * sizeof(float);
 }
@@ -802,7 +805,7 @@ extern "C" int mskv_fp8_prefill_attention_ws(
                                                          block_size, max_blocks_per_seq);
     if (workspace_bytes < need) return MSKV_EWORKSPACE;
     if (need > 0) {
-      a.splits = mskv::prefill_splits(num_seqs, max_seqlen_q, num_q_heads, num_kv_heads,
+      a.splits = mskv::prefill_splits(num_seqs, total_q, max_seqlen_q, num_q_heads, num_kv_heads,
                                       block_size, max_blocks_per_seq);
       a.part_o = (float*)workspace;
       a.part_lse = a.part_o + (size_t)total_q * num_q_heads * a.splits * head_dim;

@@ -76,6 +76,23 @@ def test_every_split_starts_within_an_int_of_tokens():
                     assert s <= w or w * block <= 1 << 22, (batch, hq, hk, w, block, s)
 
 
+def test_prefill_workspace_stays_small():
+    """The partials have a row per query row: a query tensor with more rows
+    than max_seqlen_q lets the grid cover must not ask for gigabytes."""
+    lib = _lib.load()
+    most = 0
+    for seqs in (1, 2, 8, 100):
+        for max_q in (1, 40, 512, 4096):
+            for total in (1, 40, 512, 4096, 1 << 20):
+                for hq, hk in ((32, 8), (64, 8), (40, 8), (24, 1), (8, 8)):
+                    for w in (4, 128, 4096):
+                        n = lib.mskv_fp8_prefill_workspace_bytes(seqs, total, max_q, hq, hk, 128,
+                                                                 256, w)
+                        assert n <= 35_000_000, (seqs, max_q, total, hq, hk, w, n)
+                        most = max(most, n)
+    assert most > 30_000_000
+
+
 def test_argument_validation_without_launch():
     lib = _lib.load()
     EINVAL, EUNSUP, EWS = -1, -2, -3
