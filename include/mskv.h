@@ -7,6 +7,10 @@
  * memory, synchronizes, or reads device memory on the host, so all of them
  * may be captured into a HIP graph.
  *
+ * The two prefills stage rows by 16-byte direct-to-LDS loads: their query,
+ * key, value, caches, workspace and out must start on 16 bytes, else
+ * MSKV_EINVAL.
+ *
  * Cache layout (the reference runner's, microserve/engine/model_runner.py:76-83):
  *   k_cache, v_cache           uint8 (OCP FP8 e4m3fn) [num_blocks, block_size, num_kv_heads, head_dim]
  *   k_scale_cache, v_scale_cache  float32             [num_blocks, block_size, num_kv_heads]

@@ -144,6 +144,14 @@ def store_dtype(t) -> int:
     raise AssertionError(f"key/value dtype must be float16, bfloat16 or float32, got {t.dtype}")
 
 
+def aligned(t):
+    """``t`` contiguous and on 16 bytes, as the kernels' vector loads and
+    direct-to-LDS loads read it: itself if it is, else a copy (a contiguous
+    view may start at any element)."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def token_rows(t):
     """A ``[tokens, heads, D]`` tensor and the elements between its tokens,
     for a kernel that reads whole tokens at any stride: a view with each
@@ -157,8 +165,7 @@ def token_rows(t):
         if (s2 == 1 and s1 == d and heads * d <= s0 <= 1 << 22 and s0 * size % 16 == 0
                 and t.data_ptr() % 16 == 0):
             return t, s0
-        t = t.contiguous()
-    return t, heads * d
+    return aligned(t), heads * d
 
 
 def on_device(what: str, ref, *tensors) -> None:

@@ -453,6 +453,8 @@ extern "C" int mskv_prefill_attention_strided(
   // grid y and z are limited to 65535
   const int64_t qblocks = ((int64_t)max_seqlen_q + per_wg - 1) / per_wg;
   if (num_seqs > 65535 || qblocks > 65535) return MSKV_EUNSUPPORTED;
+  // rows go to LDS directly, 16 bytes a lane
+  if (mskv::misaligned({query, key, value, out})) return MSKV_EINVAL;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (act_dtype == MSKV_BFLOAT16)
     return (int)mskv::launch_dense_sized<__bf16>(a, num_seqs, max_seqlen_q, st);

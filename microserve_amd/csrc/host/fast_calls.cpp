@@ -94,17 +94,22 @@ bool caches_match(const at::Tensor& kc, const at::Tensor& vc, const at::Tensor& 
          ks.sizes() == kc.sizes().slice(0, 3) && vs.sizes() == ks.sizes();
 }
 
+// the kernels' vector and direct-to-LDS loads start on 16 bytes
+bool aligned(const at::Tensor& t) {
+  return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+}
+
 // elements between the tokens of a [tokens, heads, D] tensor read in place
 bool token_rows(const at::Tensor& t, int64_t& stride) {
   const int64_t row = t.size(1) * t.size(2);
+  if (!aligned(t)) return false;
   if (t.is_contiguous()) {
     stride = row;
     return true;
   }
   stride = t.stride(0);
   return t.stride(2) == 1 && t.stride(1) == t.size(2) && stride >= row && stride <= 1 << 22 &&
-         stride * t.element_size() % 16 == 0 &&
-         reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+         stride * t.element_size() % 16 == 0;
 }
 
 bool number(PyObject* o, double& v) {
@@ -202,7 +207,7 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const at::Tensor* given = in.ok && a[8] != Py_None ? in.next(a[8]) : nullptr;
     double scale;
     int dt;
-    if (!in.ok || q->dim() != 3 || !q->is_contiguous() || !act(*q, dt) || !number(a[7], scale) ||
+    if (!in.ok || q->dim() != 3 || !q->is_contiguous() || !aligned(*q) || !act(*q, dt) || !number(a[7], scale) ||
         !caches_ok(*kc, *vc, *ks, *vs) || !dense_of(*len, at::kInt) || bt->dim() != 2 ||
         !dense_of(*bt, at::kInt))
       return nullptr;
@@ -263,7 +268,7 @@ PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
                      *ck = varlen && in.ok ? in.next(a[7]) : nullptr;
     double scale;
     int dt, prefix, max_q;
-    if (!in.ok || q->dim() != 3 || !q->is_contiguous() || !act(*q, dt) || !whole(a[8], prefix) ||
+    if (!in.ok || q->dim() != 3 || !q->is_contiguous() || !aligned(*q) || !act(*q, dt) || !whole(a[8], prefix) ||
         !whole(a[9], max_q) || !number(a[10], scale) || !caches_ok(*kc, *vc, *ks, *vs) ||
         !dense_of(*bt, at::kInt))
       return nullptr;
@@ -309,7 +314,7 @@ PyObject* fresh(PyObject*, PyObject* const* a, Py_ssize_t n) {
     double scale;
     int dt, max_q;
     int64_t k_stride, v_stride;
-    if (!in.ok || q->dim() != 3 || !q->is_contiguous() || !act(*q, dt) || k->dim() != 3 ||
+    if (!in.ok || q->dim() != 3 || !q->is_contiguous() || !aligned(*q) || !act(*q, dt) || k->dim() != 3 ||
         k->sizes() != v->sizes() || k->scalar_type() != q->scalar_type() ||
         v->scalar_type() != q->scalar_type() || !dense_of(*cq, at::kInt) ||
         !dense_of(*ck, at::kInt) || !whole(a[5], max_q) || !number(a[6], scale))

@@ -4,7 +4,16 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <initializer_list>
+
 namespace mskv {
+
+// Host: whether any of these pointers is not on 16 bytes (null is)
+static inline bool misaligned(std::initializer_list<const void*> pointers) {
+  for (const void* p : pointers)
+    if ((uintptr_t)p & 15u) return true;
+  return false;
+}
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));

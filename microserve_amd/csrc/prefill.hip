@@ -796,6 +796,8 @@ extern "C" int mskv_fp8_prefill_attention_ws(
   // grid y and z are limited to 65535
   const int64_t qblocks = ((int64_t)max_seqlen_q + per_wg - 1) / per_wg;
   if (num_seqs > 65535 || qblocks > 65535) return MSKV_EUNSUPPORTED;
+  // rows go to LDS directly, 16 bytes a lane
+  if (mskv::misaligned({query, k_cache, v_cache, out, workspace})) return MSKV_EINVAL;
   // without a workspace, one workgroup walks all the keys of its rows
   a.splits = 1;
   a.part_o = a.part_lse = nullptr;

@@ -70,7 +70,7 @@ def fp8_chunk_prefill_attention(
                               None, None, prefix_len, 0, softmax_scale)
     if res is not None:
         return res
-    query = query.contiguous()
+    query = _lib.aligned(query)
     block_table = block_table.contiguous().view(-1)
     query_len = query.shape[0]
     _check_common(query, k_cache, v_cache, k_scale_cache, v_scale_cache)
@@ -107,7 +107,7 @@ def fp8_varlen_prefill_attention(
                               cu_seqlens_q, cu_seqlens_k, 0, max_seqlen_q, softmax_scale)
     if res is not None:
         return res
-    query = query.contiguous()
+    query = _lib.aligned(query)
     block_tables = block_tables.contiguous()
     cu_seqlens_q = cu_seqlens_q.contiguous()
     cu_seqlens_k = cu_seqlens_k.contiguous()

@@ -83,7 +83,7 @@ def fp8_decode_attention(
                              block_tables, softmax_scale, out, _scratch)
     if res is not None:
         return res
-    query = query.contiguous()
+    query = _lib.aligned(query)
     cache_seqlens = cache_seqlens.contiguous()
     block_tables = block_tables.contiguous()
     batch_size, num_q_heads, head_dim = query.shape

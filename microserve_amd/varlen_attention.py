@@ -34,7 +34,7 @@ def varlen_attention(
                             softmax_scale if softmax_scale is not None else q.shape[-1] ** -0.5)
     if res is not None:
         return res
-    q = q.contiguous()
+    q = _lib.aligned(q)
     cu_seqlens_q = cu_seqlens_q.contiguous()
     cu_seqlens_k = cu_seqlens_k.contiguous()
     total_q, num_q_heads, head_dim = q.shape

@@ -137,6 +137,44 @@ def test_argument_validation_without_launch():
         assert lib.mskv_prefill_attention(1, 1, 1, 1, 1, 1, 1, 10, 10, 10, 32, 8, 128, sc, 1, None) == EUNSUP
 
 
+def test_prefills_reject_pointers_off_16_bytes():
+    lib = _lib.load()
+    EINVAL, A = -1, 1 << 20  # a 16-byte aligned stand-in address; nothing is launched
+
+    def paged(**off):
+        p = {k: A + off.get(k, 0) for k in ("q", "kc", "vc", "out", "ws")}
+        return lib.mskv_fp8_prefill_attention_ws(
+            p["q"], p["kc"], p["vc"], A, A, A, None, None, 0, p["out"], 1, 10, 10, 32, 8, 128,
+            256, 10, 4, 0.1, 1, p["ws"], 1 << 30, None)
+
+    def fresh(**off):
+        p = {k: A + off.get(k, 0) for k in ("q", "k", "v", "out")}
+        return lib.mskv_prefill_attention(p["q"], p["k"], p["v"], p["out"], A, A, 1, 10, 10, 10,
+                                          32, 8, 128, 0.1, 1, None)
+
+    # (without a GPU an aligned call gets as far as a launch that fails)
+    for name in ("q", "kc", "vc", "out", "ws"):
+        for by in (2, 4, 8):
+            assert paged(**{name: by}) == EINVAL
+    for name in ("q", "k", "v", "out"):
+        for by in (2, 4, 8):
+            assert fresh(**{name: by}) == EINVAL
+
+
+def test_wrappers_copy_rows_off_16_bytes():
+    import torch
+    flat = torch.arange(3 * 4 * 128 + 9).to(torch.bfloat16)
+    for at in (0, 1, 2, 4, 8):
+        view = flat[at:at + 3 * 4 * 128].view(3, 4, 128)
+        assert view.is_contiguous()
+        rows, stride = _lib.token_rows(view)
+        assert stride == 4 * 128 and rows.data_ptr() % 16 == 0
+        assert torch.equal(rows, view) and torch.equal(_lib.aligned(view), view)
+        assert _lib.aligned(view).data_ptr() % 16 == 0
+        if view.data_ptr() % 16 == 0:
+            assert rows is view
+
+
 def test_new_entry_points_validate_without_launch():
     lib = _lib.load()
     EINVAL, EUNSUP = -1, -2

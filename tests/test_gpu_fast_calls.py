@@ -79,6 +79,41 @@ def test_native_paths_give_the_wrappers_results(dtype, monkeypatch):
             _both(monkeypatch, prologue)
 
 
+@pytest.mark.parametrize("by", [1, 2])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_contiguous_inputs_off_16_bytes_give_their_copies_results(dtype, by):
+    """A contiguous view may start at any element: the kernels' 16-byte loads
+    need its copy, on the native path and on the wrappers'."""
+    gen = torch.Generator().manual_seed(821)
+    n, hq, hk = 9, 8, 2
+
+    def pair(heads):
+        flat = torch.randn(n * heads * H.D + 8, generator=gen).to(dtype).to(H.DEV)
+        view = flat[by:by + n * heads * H.D].view(n, heads, H.D)
+        assert view.is_contiguous() and view.data_ptr() % 16
+        return view, view.clone()
+
+    slots = torch.arange(300, 300 + n, device=H.DEV)
+    (k, kc), (v, vc), (q, qc) = pair(hk), pair(hk), pair(hq)
+    a, b = H.alloc_cache(4, H.BLOCK, hk), H.alloc_cache(4, H.BLOCK, hk)
+    store_fp8_kvcache(k, v, *a, slots)
+    store_fp8_kvcache(kc, vc, *b, slots)
+    for x, y in zip(a, b):
+        assert torch.equal(x.view(torch.uint8), y.view(torch.uint8))
+    if dtype == torch.float32:
+        return
+    lens = torch.full((n,), 309, dtype=torch.int32, device=H.DEV)
+    tables = torch.tensor([[0, 1]], dtype=torch.int32, device=H.DEV)
+    wide = tables.expand(n, 2).contiguous()
+    cu = torch.tensor([0, n], dtype=torch.int32, device=H.DEV)
+    ck = torch.tensor([0, 309], dtype=torch.int32, device=H.DEV)
+    for call in (lambda q, k, v: fp8_decode_attention(q, *a, lens, wide, 0.1),
+                 lambda q, k, v: fp8_chunk_prefill_attention(q, *a, tables, 300, 0.1),
+                 lambda q, k, v: fp8_varlen_prefill_attention(q, *a, tables, cu, ck, n, 0.1),
+                 lambda q, k, v: varlen_attention(q, k, v, cu, cu, n)):
+        assert torch.equal(call(q, k, v), call(qc, kc, vc))
+
+
 def test_native_paths_leave_the_rest_to_the_wrappers():
     q, k, v, slots, caches = _case(torch.float16)
     _lib.load()
