@@ -7,10 +7,12 @@
 // here takes its wrapper's arguments, and if every tensor is an ordinary one
 // that the kernel can read in place (exact class, this GPU, the dtypes,
 // shapes and strides the wrapper asserts) it allocates the outputs and calls
-// the C ABI directly.  Anything else, an error status included, returns
-// None before or without effect, and the wrapper's own path, the only place
-// where arguments are converted and errors raised, runs as if this module
-// did not exist.  (A call that is repeated writes the same values.)
+// the C ABI directly.  Anything else, arguments that the C ABI rejects
+// included (a negative status, before any launch), returns None without
+// effect, and the wrapper's own path, the only place where arguments are
+// converted and checked, runs as if this module did not exist.  A launch
+// that failed (a positive status) raises here: the runtime forgets an error
+// once it has been read, so a second try could pass in silence.
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
@@ -30,6 +32,7 @@ struct Api {
   decltype(&mskv_fp8_prefill_attention_ws) prefill = nullptr;
   decltype(&mskv_prefill_attention_strided) fresh = nullptr;
   decltype(&mskv_qk_norm_rope_store) prologue = nullptr;
+  decltype(&mskv_status_string) text = nullptr;
   bool bound = false;
 } api;
 
@@ -162,6 +165,14 @@ PyObject* guarded(F&& f) {
   Py_RETURN_NONE;
 }
 
+// A call's non-zero status: null without an error if the arguments were
+// rejected, else with the wrapper's error.
+PyObject* failed(const char* what, int status) {
+  if (status > 0)
+    PyErr_Format(PyExc_RuntimeError, "%s failed: status %d (%s)", what, status, api.text(status));
+  return nullptr;
+}
+
 // store(key, value, k_cache, v_cache, k_scale, v_scale, slots) -> True | None
 PyObject* store(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
@@ -189,7 +200,7 @@ PyObject* store(PyObject*, PyObject* const* a, Py_ssize_t n) {
                   st, key->size(0), (int)key->size(1), (int)key->size(2),
                   kc->size(0) * kc->size(1), dt, stream_of(in.device));
     }
-    if (status != MSKV_OK) return nullptr;
+    if (status != MSKV_OK) return failed("store_fp8_kvcache", status);
     Py_RETURN_TRUE;
   });
 }
@@ -245,7 +256,7 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
                    out.data_ptr(), (int)b, (int)hq, (int)hk, (int)d, (int)bs, kc->size(0), (int)w,
                    (float)scale, dt, splits, ws, bytes, stream);
     }
-    if (status != MSKV_OK) return nullptr;
+    if (status != MSKV_OK) return failed("fp8_decode_attention", status);
     if (given) {
       Py_INCREF(a[8]);
       return a[8];
@@ -299,7 +310,9 @@ PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
                     (float)scale, dt, bytes ? ws.data_ptr() : nullptr, bytes,
                     stream_of(in.device));
     }
-    if (status != MSKV_OK) return nullptr;
+    if (status != MSKV_OK)
+      return failed(varlen ? "fp8_varlen_prefill_attention" : "fp8_chunk_prefill_attention",
+                    status);
     return THPVariable_Wrap(std::move(out));
   });
 }
@@ -333,7 +346,7 @@ PyObject* fresh(PyObject*, PyObject* const* a, Py_ssize_t n) {
                   (int32_t*)cq->data_ptr(), (int32_t*)ck->data_ptr(), (int)seqs, nq, nk, max_q,
                   (int)hq, (int)hk, (int)d, (float)scale, dt, stream_of(in.device));
     }
-    if (status != MSKV_OK) return nullptr;
+    if (status != MSKV_OK) return failed("varlen_attention", status);
     return THPVariable_Wrap(std::move(out));
   });
 }
@@ -387,7 +400,7 @@ PyObject* prologue(PyObject*, PyObject* const* a, Py_ssize_t n) {
                      (float*)vs->data_ptr(), sl->data_ptr(), st, t, (int)hq, (int)hk, (int)d,
                      kc->size(0) * kc->size(1), dt, stream_of(in.device));
     }
-    if (status != MSKV_OK) return nullptr;
+    if (status != MSKV_OK) return failed("mskv_qk_norm_rope_store", status);
     PyObject* qo = THPVariable_Wrap(std::move(q_out));
     PyObject* ko = Py_None;
     if (with_k)
@@ -415,7 +428,7 @@ PyObject* bind(PyObject*, PyObject* table) {
             get("mskv_fp8_prefill_workspace_bytes", f.prefill_bytes) &&
             get("mskv_fp8_prefill_attention_ws", f.prefill) &&
             get("mskv_prefill_attention_strided", f.fresh) &&
-            get("mskv_qk_norm_rope_store", f.prologue);
+            get("mskv_qk_norm_rope_store", f.prologue) && get("mskv_status_string", f.text);
   if (!f.bound) {
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_KeyError, "an entry point has no address");
     return nullptr;

@@ -1,6 +1,8 @@
 """The native call paths take ordinary calls, give the wrappers' own results
 bit for bit, and leave everything else to the wrappers."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -150,3 +152,51 @@ def test_native_paths_leave_the_rest_to_the_wrappers():
     with pytest.raises(RuntimeError, match="status -2"):
         varlen_attention(q.contiguous(), k, v, lens[:2].cumsum(0, dtype=torch.int32) - 1,
                          lens[:2].cumsum(0, dtype=torch.int32) - 1, 1, softmax_scale=-1.0)
+
+
+def test_a_failed_launch_raises_and_is_not_tried_again():
+    """A positive status is a HIP error that the runtime has already
+    forgotten: the native path raises it as the wrapper would, and nothing
+    calls the entry point a second time.  (The entry points are stood in for
+    by a host function; no kernel runs.)"""
+    q, k, v, slots, caches = _case(torch.float16)
+    lib = _lib.load()
+    real = {n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in _lib.EXPORTED}
+    calls = []
+
+    @ctypes.CFUNCTYPE(ctypes.c_int)
+    def stub():
+        calls.append(1)
+        return 719
+
+    address = ctypes.cast(stub, ctypes.c_void_p).value
+    entries = ("mskv_store_fp8_kvcache_strided", "mskv_fp8_decode_attention",
+               "mskv_fp8_prefill_attention_ws", "mskv_prefill_attention_strided",
+               "mskv_qk_norm_rope_store")
+    qc = q.contiguous()
+    lens = torch.ones(5, dtype=torch.int32, device=H.DEV)
+    tables = torch.zeros(5, 1, dtype=torch.int32, device=H.DEV)
+    cu = torch.tensor([0, 5], dtype=torch.int32, device=H.DEV)
+    cos, sin = (torch.randn(64, H.D, device=H.DEV).half() for _ in range(2))
+    pos = torch.arange(5, device=H.DEV)
+    _lib.fast.bind({**real, **{n: address for n in entries}})
+    try:
+        for what, call in (
+                ("store_fp8_kvcache", lambda: store_fp8_kvcache(k, v, *caches, slots)),
+                ("fp8_decode_attention",
+                 lambda: fp8_decode_attention(qc, *caches, lens, tables, 0.1)),
+                ("fp8_chunk_prefill_attention",
+                 lambda: fp8_chunk_prefill_attention(qc, *caches, tables[:1], 3, 0.1)),
+                ("fp8_varlen_prefill_attention",
+                 lambda: fp8_varlen_prefill_attention(qc, *caches, tables[:1], cu, cu, 5, 0.1)),
+                ("varlen_attention", lambda: varlen_attention(qc, k, v, cu, cu, 5)),
+                ("mskv_qk_norm_rope_store",
+                 lambda: qk_norm_rope_store(pos, q, k, v, None, None, 1e-6, cos, sin, *caches,
+                                            slots))):
+            calls.clear()
+            with pytest.raises(RuntimeError, match=rf"{what} failed: status 719 \("):
+                call()
+            assert len(calls) == 1
+    finally:
+        _lib.fast.bind(real)
+    assert torch.isfinite(fp8_decode_attention(qc, *caches, lens, tables, 0.1).float()).all()
