@@ -15,21 +15,39 @@ import os
 import torch  # noqa: F401  (the extension below uses its libraries)
 
 
-class _NotBuilt:
-    """Stands in for the native call paths until they are built (the package
-    must import to be built): raises on use."""
+_FAST = "microserve_amd._fast_calls"
+
+
+class _Missing:
+    """Stands in for the native call paths while they cannot be imported (the
+    package must import to be built).  Every use looks for them again, since
+    they may have been built meanwhile, and raises if they are still not
+    there: not built, or built but not loadable, with the cause."""
 
     def __getattr__(self, name):
-        raise RuntimeError("microserve_amd._fast_calls is not built: run "
-                           "`python -m microserve_amd.build`")
+        global fast
+        found = _import_fast()
+        if isinstance(found, _Missing):
+            cause = vars(found)["cause"]
+            if isinstance(cause, ModuleNotFoundError) and cause.name == _FAST:
+                raise RuntimeError(f"{_FAST} is not built: run "
+                                   "`python -m microserve_amd.build`") from cause
+            raise RuntimeError(f"{_FAST} cannot be loaded ({cause}); if it was built against "
+                               "another torch, run `python -m microserve_amd.build`") from cause
+        fast = found
+        if _lib is not None:
+            _bind(_lib)
+        return getattr(fast, name)
 
 
 def _import_fast():
     importlib.invalidate_caches()
     try:
-        return importlib.import_module("microserve_amd._fast_calls")
-    except ImportError:
-        return _NotBuilt()
+        return importlib.import_module(_FAST)
+    except ImportError as e:
+        missing = _Missing()
+        vars(missing)["cause"] = e
+        return missing
 
 
 fast = _import_fast()
@@ -98,7 +116,7 @@ _lib = None
 
 def load() -> ctypes.CDLL:
     """Load libmskv.so once; raise with a build hint if it is absent."""
-    global _lib, fast
+    global _lib
     if _lib is not None:
         return _lib
     if not os.path.exists(LIB_PATH):
@@ -110,11 +128,14 @@ def load() -> ctypes.CDLL:
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
-    if isinstance(fast, _NotBuilt):  # built since this module was imported
-        fast = _import_fast()
-    fast.bind({name: ctypes.cast(getattr(lib, name), _vp).value for name in _PROTOS})
+    if not isinstance(fast, _Missing):  # (the library needs only itself)
+        _bind(lib)
     _lib = lib
     return lib
+
+
+def _bind(lib) -> None:
+    fast.bind({name: ctypes.cast(getattr(lib, name), _vp).value for name in _PROTOS})
 
 
 def check(status: int, what: str) -> None:

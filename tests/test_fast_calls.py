@@ -1,6 +1,9 @@
 """The native call paths leave every call they cannot take as it stands to
 the wrappers: on the CPU, tensors that are not on a GPU."""
 
+import importlib
+
+import pytest
 import torch
 
 from microserve_amd import _lib
@@ -33,3 +36,41 @@ def test_wrong_argument_counts_and_types_are_left_to_the_wrappers():
     for fn in (f.store, f.decode, f.prefill, f.fresh, f.prologue):
         assert fn() is None
         assert fn(*[None] * 7) is None and fn(*["x"] * 15) is None and fn(*[3] * 10) is None
+
+
+def _without_extension(monkeypatch, error):
+    """A process in which importing the extension raises `error`."""
+    real = importlib.import_module
+
+    def fail(name, *a):
+        if name == _lib._FAST:
+            raise error
+        return real(name, *a)
+
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "fast", _lib.fast)
+    monkeypatch.setattr(importlib, "import_module", fail)
+    _lib.fast = _lib._import_fast()
+    return real
+
+
+def test_an_extension_that_does_not_load_names_its_cause(monkeypatch):
+    cause = ImportError("undefined symbol: _ZN3c105ErrorE")
+    _without_extension(monkeypatch, cause)
+    with pytest.raises(RuntimeError, match="undefined symbol: _ZN3c105ErrorE") as e:
+        _lib.fast.decode()
+    assert e.value.__cause__ is cause and "not built" not in str(e.value)
+
+
+def test_an_extension_built_later_is_found_by_the_next_call(monkeypatch):
+    real = _without_extension(monkeypatch, ModuleNotFoundError(name=_lib._FAST))
+    with pytest.raises(RuntimeError, match="not built"):
+        _lib.fast.decode()
+    monkeypatch.setattr(importlib, "import_module", real)
+    assert _lib.fast.decode() is None
+    assert _lib.fast is real(_lib._FAST)
+
+
+def test_the_library_loads_without_the_extension(monkeypatch):
+    _without_extension(monkeypatch, ModuleNotFoundError(name=_lib._FAST))
+    assert _lib.load().mskv_version() >= 100
