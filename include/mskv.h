@@ -239,6 +239,26 @@ int mskv_fp8_prefill_attention_ws(const void* query, const void* k_cache,
                                   size_t workspace_bytes, void* stream);
 
 /*
+ * Both, given a bound of the keys that any sequence has (0: unknown, the
+ * width of its table).  It chooses the number of key ranges and nothing else:
+ * results hold for every key count, but a bound far above the keys pays for
+ * a merge of nothing, one below them leaves their ranges longer.
+ */
+size_t mskv_fp8_prefill_bounded_workspace_bytes(
+    int num_seqs, int64_t total_q, int max_seqlen_q, int64_t max_seqlen_k,
+    int num_q_heads, int num_kv_heads, int head_dim, int block_size,
+    int max_blocks_per_seq);
+int mskv_fp8_prefill_attention_bounded(
+    const void* query, const void* k_cache, const void* v_cache,
+    const float* k_scale_cache, const float* v_scale_cache,
+    const int32_t* block_tables, const int32_t* cu_seqlens_q,
+    const int32_t* cu_seqlens_k, int prefix_len, void* out, int num_seqs,
+    int64_t total_q, int max_seqlen_q, int64_t max_seqlen_k, int num_q_heads,
+    int num_kv_heads, int head_dim, int block_size, int64_t num_blocks,
+    int max_blocks_per_seq, float softmax_scale, int act_dtype,
+    void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Causal varlen attention over unquantized q/k/v: the fresh PREFILL of the
  * FP8-KV path.
  *

@@ -94,6 +94,12 @@ _PROTOS = {
         _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_int, _vp,
         _c_int, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_i64,
         _c_int, _c_f32, _c_int, _vp, _c_size, _vp]),
+    "mskv_fp8_prefill_bounded_workspace_bytes": (_c_size, [
+        _c_int, _c_i64, _c_int, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int]),
+    "mskv_fp8_prefill_attention_bounded": (_c_int, [
+        _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_int, _vp,
+        _c_int, _c_i64, _c_int, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_i64,
+        _c_int, _c_f32, _c_int, _vp, _c_size, _vp]),
     "mskv_prefill_attention": (_c_int, [
         _vp, _vp, _vp, _vp, _vp, _vp, _c_int, _c_i64, _c_i64, _c_int,
         _c_int, _c_int, _c_int, _c_f32, _c_int, _vp]),

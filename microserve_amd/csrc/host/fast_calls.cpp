@@ -28,8 +28,8 @@ struct Api {
   decltype(&mskv_decode_num_splits) num_splits = nullptr;
   decltype(&mskv_decode_workspace_bytes) decode_bytes = nullptr;
   decltype(&mskv_fp8_decode_attention) decode = nullptr;
-  decltype(&mskv_fp8_prefill_workspace_bytes) prefill_bytes = nullptr;
-  decltype(&mskv_fp8_prefill_attention_ws) prefill = nullptr;
+  decltype(&mskv_fp8_prefill_bounded_workspace_bytes) prefill_bytes = nullptr;
+  decltype(&mskv_fp8_prefill_attention_bounded) prefill = nullptr;
   decltype(&mskv_prefill_attention_strided) fresh = nullptr;
   decltype(&mskv_qk_norm_rope_store) prologue = nullptr;
   decltype(&mskv_status_string) text = nullptr;
@@ -266,11 +266,12 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // prefill(query, k_cache, v_cache, k_scale, v_scale, tables, cu_q | None,
-//         cu_k | None, prefix_len, max_seqlen_q, scale) -> out | None
-// (without cu_q, one sequence: max_seqlen_q is not read)
+//         cu_k | None, prefix_len, max_seqlen_q, max_seqlen_k, scale)
+//   -> out | None
+// (without cu_q, one sequence: max_seqlen_q and max_seqlen_k are not read)
 PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
-    if (n != 11) return nullptr;
+    if (n != 12) return nullptr;
     Args in;
     const at::Tensor *q = in.first(a[0]), *kc = in.next(a[1]), *vc = in.next(a[2]),
                      *ks = in.next(a[3]), *vs = in.next(a[4]), *bt = in.next(a[5]);
@@ -278,9 +279,9 @@ PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const at::Tensor *cq = varlen && in.ok ? in.next(a[6]) : nullptr,
                      *ck = varlen && in.ok ? in.next(a[7]) : nullptr;
     double scale;
-    int dt, prefix, max_q;
+    int dt, prefix, max_q, bound;
     if (!in.ok || q->dim() != 3 || !q->is_contiguous() || !aligned(*q) || !act(*q, dt) || !whole(a[8], prefix) ||
-        !whole(a[9], max_q) || !number(a[10], scale) || !caches_ok(*kc, *vc, *ks, *vs) ||
+        !whole(a[9], max_q) || !whole(a[10], bound) || !number(a[11], scale) || !caches_ok(*kc, *vc, *ks, *vs) ||
         !dense_of(*bt, at::kInt))
       return nullptr;
     const int64_t nq = q->size(0), hq = q->size(1), d = q->size(2), hk = kc->size(2),
@@ -293,9 +294,13 @@ PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
       if (ck->numel() != seqs + 1 || bt->size(0) != seqs) return nullptr;
     }
     if (!fits({nq, hq, d, hk, bs, w, seqs}) || hq % hk != 0 || d != kc->size(3)) return nullptr;
-    if (!varlen) max_q = (int)nq;
-    const size_t bytes = api.prefill_bytes((int)seqs, nq, max_q, (int)hq, (int)hk, (int)d, (int)bs,
-                                           (int)w);
+    int64_t max_k = bound;
+    if (!varlen) {
+      max_q = (int)nq;
+      max_k = prefix + nq;
+    }
+    const size_t bytes = api.prefill_bytes((int)seqs, nq, max_q, max_k, (int)hq, (int)hk, (int)d,
+                                           (int)bs, (int)w);
     at::Tensor ws, out;
     int status;
     {
@@ -306,7 +311,7 @@ PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
                     (float*)vs->data_ptr(), (int32_t*)bt->data_ptr(),
                     varlen ? (int32_t*)cq->data_ptr() : nullptr,
                     varlen ? (int32_t*)ck->data_ptr() : nullptr, prefix, out.data_ptr(), (int)seqs,
-                    nq, max_q, (int)hq, (int)hk, (int)d, (int)bs, kc->size(0), (int)w,
+                    nq, max_q, max_k, (int)hq, (int)hk, (int)d, (int)bs, kc->size(0), (int)w,
                     (float)scale, dt, bytes ? ws.data_ptr() : nullptr, bytes,
                     stream_of(in.device));
     }
@@ -425,8 +430,8 @@ PyObject* bind(PyObject*, PyObject* table) {
             get("mskv_decode_num_splits", f.num_splits) &&
             get("mskv_decode_workspace_bytes", f.decode_bytes) &&
             get("mskv_fp8_decode_attention", f.decode) &&
-            get("mskv_fp8_prefill_workspace_bytes", f.prefill_bytes) &&
-            get("mskv_fp8_prefill_attention_ws", f.prefill) &&
+            get("mskv_fp8_prefill_bounded_workspace_bytes", f.prefill_bytes) &&
+            get("mskv_fp8_prefill_attention_bounded", f.prefill) &&
             get("mskv_prefill_attention_strided", f.fresh) &&
             get("mskv_qk_norm_rope_store", f.prologue) && get("mskv_status_string", f.text);
   if (!f.bound) {

@@ -49,6 +49,8 @@
 #include <float.h>
 #include <math.h>
 
+#include <algorithm>
+
 #include "mskv_device.h"
 #include "../../include/mskv.h"
 
@@ -676,7 +678,7 @@ static hipError_t launch_prefill(const PrefillArgs& a, int num_seqs, int64_t qbl
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   // the tokens of a sequence that the grid covers
-  const int tokens = (int)min(qblocks * 8 * a.tpr, a.total_q);
+  const int tokens = (int)std::min(qblocks * 8 * a.tpr, a.total_q);
   switch (a.splits) {
     case 2: launch_merge<T, 2>(a, num_seqs, tokens, st); break;
     case 3: launch_merge<T, 3>(a, num_seqs, tokens, st); break;
@@ -689,34 +691,45 @@ static hipError_t launch_prefill(const PrefillArgs& a, int num_seqs, int64_t qbl
   return hipGetLastError();
 }
 
-// Key ranges per workgroup, from shapes alone.  Two workgroups are resident
-// per CU, 512 on the chip, and a second one costs the first little (a tile
-// takes 3.2 us alone, 3.9 us beside another), so a grid of at most 256 is
-// split until it fills them (768 or 1024 instead: 120-134 against 106 us on
-// 512 new over 7680 cached tokens), where the shorter chain saves more than
-// the merge costs: its launch, 5 us, and 1 KB per row and split at 6 TB/s.
-// Unsplit against split (fp16, 32 q / 8 kv heads, new/cached, with the
-// store, us): 512/7680 210 -> 106, 128/7680 195 -> 53, 64/2000 66 -> 31,
-// 512/1000 54 -> 46, 256/600 39 -> 35; split all the same, 4 x 74/129 went
-// 12.5 -> 18.0 and 509/200 at 64 q heads 33.8 -> 35.8.
+// Key ranges per workgroup, from what the host knows: the shapes and a bound
+// of a sequence's keys (the call's own, or the table's width).  Two
+// workgroups are resident per CU, 512 on the chip, and a second one costs the
+// first little (a tile takes 3.0 us unsplit, 3.2 us beside other ranges, 3.9
+// us beside another workgroup), so a grid of at most 256 is split until it
+// fills them (768 or 1024 instead: 120-134 against 106 us on 512 new over
+// 7680 cached tokens, with the store), where the shorter chain saves more
+// than the merge costs: its launch, 5 us, and 1 KB per row and split at 6
+// TB/s.  Unsplit against split (fp16, 32 q / 8 kv heads, new/cached, the
+// call alone, us): 512/7680 191 -> 83, 128/7680 182 -> 41, 512/1000 42.2 ->
+// 36.0, 128/600 24.9 -> 20.4; left unsplit, 512/300 28.2 (2 splits 30.7, 4
+// 31.4), 256/300 22.4 (8 splits 28.4), 128/300 19.3 (19.5), 4 x 74/129 13.6
+// (16.5).  Hence also the bound: by the width of a table of 128 pages, the
+// last three and 256 new tokens alone (13.2 unsplit, 18.2) would be split.
 // The partials hold every row of the query tensor: one with more rows than
 // the grid covers (a padded one, its max_seqlen_q that of the real tokens)
 // is not split, so that they stay below 512 workgroups' rows.
-static int prefill_splits(int num_seqs, int64_t total_q, int64_t max_seqlen_q, int num_q_heads,
-                          int num_kv_heads, int block_size, int max_blocks_per_seq) {
+static int prefill_splits(int num_seqs, int64_t total_q, int64_t max_seqlen_q,
+                          int64_t max_seqlen_k, int num_q_heads, int num_kv_heads, int block_size,
+                          int max_blocks_per_seq) {
   const int group = num_q_heads / num_kv_heads;
   const int per_wg = 8 * (group < 16 ? 16 / group : 1);
   const int64_t qblocks = (max_seqlen_q + per_wg - 1) / per_wg;
   const int64_t wgs = num_seqs * qblocks * num_kv_heads * ((group + 15) / 16);
   if (wgs <= 0 || wgs > 512 || total_q * num_q_heads > wgs * 8 * 16) return 1;
-  const int64_t tiles = (int64_t)max_blocks_per_seq * block_size / kPStep;
-  const int64_t most =
-      min(min((int64_t)512 / wgs, tiles / kPMinSplitTiles), (int64_t)kPMaxSplits);
+  // whole pages, so that a bound says what a table just wide enough says: one
+  // sequence's chunk has the same bits with either
+  // (std::min: on the host, HIP's min takes ints)
+  int64_t pages = max_blocks_per_seq;
+  if (max_seqlen_k > 0) pages = std::min(pages, (max_seqlen_k - 1) / block_size + 1);
+  const int64_t tiles = pages * block_size / kPStep;
+  const int64_t most = std::min({512 / wgs, tiles / kPMinSplitTiles, (int64_t)kPMaxSplits});
   const double rows = (double)wgs * 8 * 16;
   int best = 1;
-  double best_saved = 2.0;  // us: the table bounds the keys from above only
+  double best_saved = 2.0;  // us: the bound is one from above only
   for (int s = 2; s <= most; ++s) {
-    const double saved = 3.2 * (double)(tiles - (tiles + s - 1) / s) - 5.0 - rows * s * 1.7e-4;
+    const double tile = wgs * s <= 256 ? 3.2 : 3.9;
+    const double saved =
+        3.0 * (double)tiles - tile * (double)((tiles + s - 1) / s) - 5.0 - rows * s * 1.7e-4;
     if (saved > best_saved) {
       best = s;
       best_saved = saved;
@@ -727,25 +740,33 @@ static int prefill_splits(int num_seqs, int64_t total_q, int64_t max_seqlen_q, i
 
 }  // namespace mskv
 
-extern "C" size_t mskv_fp8_prefill_workspace_bytes(int num_seqs, int64_t total_q, int max_seqlen_q,
-                                                   int num_q_heads, int num_kv_heads,
-                                                   int head_dim, int block_size,
-                                                   int max_blocks_per_seq) {
+extern "C" size_t mskv_fp8_prefill_bounded_workspace_bytes(
+    int num_seqs, int64_t total_q, int max_seqlen_q, int64_t max_seqlen_k, int num_q_heads,
+    int num_kv_heads, int head_dim, int block_size, int max_blocks_per_seq) {
   if (num_seqs <= 0 || total_q <= 0 || max_seqlen_q <= 0 || num_q_heads <= 0 ||
       num_kv_heads <= 0 || num_q_heads % num_kv_heads != 0 || head_dim != mskv::kHeadDim ||
       block_size <= 0 || block_size % mskv::kPStep != 0 || max_blocks_per_seq <= 0)
     return 0;
-  const int s = mskv::prefill_splits(num_seqs, total_q, max_seqlen_q, num_q_heads, num_kv_heads,
-                                     block_size, max_blocks_per_seq);
+  const int s = mskv::prefill_splits(num_seqs, total_q, max_seqlen_q, max_seqlen_k, num_q_heads,
+                                     num_kv_heads, block_size, max_blocks_per_seq);
   return s < 2 ? 0 : (size_t)total_q * num_q_heads * s * (mskv::kHeadDim + 1) * sizeof(float);
 }
 
-extern "C" int mskv_fp8_prefill_attention_ws(
+extern "C" size_t mskv_fp8_prefill_workspace_bytes(int num_seqs, int64_t total_q, int max_seqlen_q,
+                                                   int num_q_heads, int num_kv_heads,
+                                                   int head_dim, int block_size,
+                                                   int max_blocks_per_seq) {
+  return mskv_fp8_prefill_bounded_workspace_bytes(num_seqs, total_q, max_seqlen_q, 0, num_q_heads,
+                                                  num_kv_heads, head_dim, block_size,
+                                                  max_blocks_per_seq);
+}
+
+extern "C" int mskv_fp8_prefill_attention_bounded(
     const void* query, const void* k_cache, const void* v_cache,
     const float* k_scale_cache, const float* v_scale_cache,
     const int32_t* block_tables, const int32_t* cu_seqlens_q,
     const int32_t* cu_seqlens_k, int prefix_len, void* out, int num_seqs,
-    int64_t total_q, int max_seqlen_q, int num_q_heads, int num_kv_heads,
+    int64_t total_q, int max_seqlen_q, int64_t max_seqlen_k, int num_q_heads, int num_kv_heads,
     int head_dim, int block_size, int64_t num_blocks, int max_blocks_per_seq,
     float softmax_scale, int act_dtype, void* workspace, size_t workspace_bytes,
     void* stream) {
@@ -802,13 +823,13 @@ extern "C" int mskv_fp8_prefill_attention_ws(
   a.splits = 1;
   a.part_o = a.part_lse = nullptr;
   if (workspace) {
-    const size_t need = mskv_fp8_prefill_workspace_bytes(num_seqs, total_q, max_seqlen_q,
-                                                         num_q_heads, num_kv_heads, head_dim,
-                                                         block_size, max_blocks_per_seq);
+    const size_t need = mskv_fp8_prefill_bounded_workspace_bytes(
+        num_seqs, total_q, max_seqlen_q, max_seqlen_k, num_q_heads, num_kv_heads, head_dim,
+        block_size, max_blocks_per_seq);
     if (workspace_bytes < need) return MSKV_EWORKSPACE;
     if (need > 0) {
-      a.splits = mskv::prefill_splits(num_seqs, total_q, max_seqlen_q, num_q_heads, num_kv_heads,
-                                      block_size, max_blocks_per_seq);
+      a.splits = mskv::prefill_splits(num_seqs, total_q, max_seqlen_q, max_seqlen_k, num_q_heads,
+                                      num_kv_heads, block_size, max_blocks_per_seq);
       a.part_o = (float*)workspace;
       a.part_lse = a.part_o + (size_t)total_q * num_q_heads * a.splits * head_dim;
     }
@@ -817,6 +838,22 @@ extern "C" int mskv_fp8_prefill_attention_ws(
   if (act_dtype == MSKV_BFLOAT16)
     return (int)mskv::launch_prefill<__bf16>(a, num_seqs, qblocks, s);
   return (int)mskv::launch_prefill<_Float16>(a, num_seqs, qblocks, s);
+}
+
+extern "C" int mskv_fp8_prefill_attention_ws(
+    const void* query, const void* k_cache, const void* v_cache,
+    const float* k_scale_cache, const float* v_scale_cache,
+    const int32_t* block_tables, const int32_t* cu_seqlens_q,
+    const int32_t* cu_seqlens_k, int prefix_len, void* out, int num_seqs,
+    int64_t total_q, int max_seqlen_q, int num_q_heads, int num_kv_heads,
+    int head_dim, int block_size, int64_t num_blocks, int max_blocks_per_seq,
+    float softmax_scale, int act_dtype, void* workspace, size_t workspace_bytes,
+    void* stream) {
+  return mskv_fp8_prefill_attention_bounded(
+      query, k_cache, v_cache, k_scale_cache, v_scale_cache, block_tables, cu_seqlens_q,
+      cu_seqlens_k, prefix_len, out, num_seqs, total_q, max_seqlen_q, 0, num_q_heads, num_kv_heads,
+      head_dim, block_size, num_blocks, max_blocks_per_seq, softmax_scale, act_dtype, workspace,
+      workspace_bytes, stream);
 }
 
 extern "C" int mskv_fp8_prefill_attention(

@@ -24,7 +24,7 @@ def _check_common(query, k_cache, v_cache, k_scale_cache, v_scale_cache):
 
 
 def _launch(lib, what, query, caches, tables, cu_q, cu_k, prefix_len, output, num_seqs,
-            max_seqlen_q, max_blocks, softmax_scale):
+            max_seqlen_q, max_seqlen_k, max_blocks, softmax_scale):
     """One prefill launch.  The split partials' workspace, where the shapes
     need one, is allocated per call on the current stream, which the kernels
     run on: the caching allocator reuses it in stream order, and a graph
@@ -32,16 +32,17 @@ def _launch(lib, what, query, caches, tables, cu_q, cu_k, prefix_len, output, nu
     k_cache, v_cache, k_scale_cache, v_scale_cache = caches
     total_q, num_q_heads, head_dim = query.shape
     num_blocks, block_size, num_kv_heads = k_cache.shape[:3]
-    ws_bytes = lib.mskv_fp8_prefill_workspace_bytes(
-        num_seqs, total_q, max_seqlen_q, num_q_heads, num_kv_heads, head_dim, block_size,
-        max_blocks)
+    ws_bytes = lib.mskv_fp8_prefill_bounded_workspace_bytes(
+        num_seqs, total_q, max_seqlen_q, max_seqlen_k, num_q_heads, num_kv_heads, head_dim,
+        block_size, max_blocks)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=query.device) if ws_bytes else None
-    status = lib.mskv_fp8_prefill_attention_ws(
+    status = lib.mskv_fp8_prefill_attention_bounded(
         query.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
         k_scale_cache.data_ptr(), v_scale_cache.data_ptr(), tables.data_ptr(),
         None if cu_q is None else cu_q.data_ptr(), None if cu_k is None else cu_k.data_ptr(),
-        prefix_len, output.data_ptr(), num_seqs, total_q, max_seqlen_q, num_q_heads,
-        num_kv_heads, head_dim, block_size, num_blocks, max_blocks, float(softmax_scale),
+        prefix_len, output.data_ptr(), num_seqs, total_q, max_seqlen_q, max_seqlen_k,
+        num_q_heads, num_kv_heads, head_dim, block_size, num_blocks, max_blocks,
+        float(softmax_scale),
         _lib.act_dtype(query), None if ws is None else ws.data_ptr(), ws_bytes,
         _lib.stream_of(query))
     _lib.check(status, what)
@@ -67,7 +68,7 @@ def fp8_chunk_prefill_attention(
     """
     del block_m, block_n
     res = _lib.fast.prefill(query, k_cache, v_cache, k_scale_cache, v_scale_cache, block_table,
-                              None, None, prefix_len, 0, softmax_scale)
+                              None, None, prefix_len, 0, 0, softmax_scale)
     if res is not None:
         return res
     query = _lib.aligned(query)
@@ -83,7 +84,8 @@ def fp8_chunk_prefill_attention(
         return output
     _launch(_lib.load(), "fp8_chunk_prefill_attention", query,
             (k_cache, v_cache, k_scale_cache, v_scale_cache), block_table, None, None, prefix_len,
-            output, 1, query_len, block_table.numel(), softmax_scale)
+            output, 1, query_len, prefix_len + query_len, block_table.numel(),
+            softmax_scale)
     return output
 
 
@@ -92,6 +94,7 @@ def fp8_varlen_prefill_attention(
     k_scale_cache: torch.Tensor, v_scale_cache: torch.Tensor,
     block_tables: torch.Tensor, cu_seqlens_q: torch.Tensor,
     cu_seqlens_k: torch.Tensor, max_seqlen_q: int, softmax_scale: float,
+    max_seqlen_k: int | None = None,
 ) -> torch.Tensor:
     """Varlen causal prefill with cached prefixes, in one launch.
 
@@ -101,10 +104,16 @@ def fp8_varlen_prefill_attention(
     cu_seqlens_k[s]`` cached positions (its new tokens included, since they
     are stored first); query ``i`` sees positions ``< Lk - Lq + i + 1``.
     ``block_tables`` is int32 ``[num_seqs, max_blocks]``.  ``max_seqlen_q``
-    is a host integer, as in the reference's ``Context``.
+    is a host integer, as in the reference's ``Context``.  ``max_seqlen_k``,
+    the most cached positions of any sequence, only chooses how many ranges
+    small batches split the keys into; without it the tables' width stands
+    in, which costs short sequences under much wider tables a few
+    microseconds (16 x 8 new over 100 cached tokens: 11.9 against 8.8).
     """
+    bound = 0 if max_seqlen_k is None else int(max_seqlen_k)
     res = _lib.fast.prefill(query, k_cache, v_cache, k_scale_cache, v_scale_cache, block_tables,
-                              cu_seqlens_q, cu_seqlens_k, 0, max_seqlen_q, softmax_scale)
+                              cu_seqlens_q, cu_seqlens_k, 0, max_seqlen_q, bound,
+                              softmax_scale)
     if res is not None:
         return res
     query = _lib.aligned(query)
@@ -124,6 +133,6 @@ def fp8_varlen_prefill_attention(
         return output
     _launch(_lib.load(), "fp8_varlen_prefill_attention", query,
             (k_cache, v_cache, k_scale_cache, v_scale_cache), block_tables, cu_seqlens_q,
-            cu_seqlens_k, 0, output, num_seqs, int(max_seqlen_q), block_tables.shape[1],
-            softmax_scale)
+            cu_seqlens_k, 0, output, num_seqs, int(max_seqlen_q), max(bound, 0),
+            block_tables.shape[1], softmax_scale)
     return output

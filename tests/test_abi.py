@@ -93,6 +93,28 @@ def test_prefill_workspace_stays_small():
     assert most > 30_000_000
 
 
+def test_prefill_splits_follow_the_bound_of_the_keys():
+    lib = _lib.load()
+
+    def ws(keys, new=40, seqs=1, w=64, heads=(32, 8)):
+        return lib.mskv_fp8_prefill_bounded_workspace_bytes(seqs, seqs * new, new, keys, *heads,
+                                                            128, 256, w)
+
+    # short contexts are not split, however wide their table
+    for w in (2, 64, 128):
+        assert ws(340, w=w) == 0 and ws(203, new=74, seqs=4, w=w) == 0
+        assert ws(812, new=512, w=max(w, 4)) == 0 and ws(256, new=256, w=w) == 0
+    # no bound, or one past the table: the table's width, as the unbounded query
+    for keys in (0, -1, 64 * 256, 1 << 40):
+        assert ws(keys) == lib.mskv_fp8_prefill_workspace_bytes(1, 40, 40, 32, 8, 128, 256, 64) > 0
+    # any bound inside the last page says what the table just wide enough says
+    for pages in (3, 5, 8, 31):
+        want = ws(0, w=pages)
+        assert want > 0
+        for keys in (256 * pages, 256 * pages - 1, 256 * pages - 255):
+            assert ws(keys) == want
+
+
 def test_argument_validation_without_launch():
     lib = _lib.load()
     EINVAL, EUNSUP, EWS = -1, -2, -3

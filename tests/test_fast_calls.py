@@ -24,7 +24,7 @@ def test_tensors_off_the_gpu_are_left_to_the_wrappers():
     f = _lib.fast
     assert f.store(k, k, kc, kc, ks, ks, i32) is None
     assert f.decode(q, kc, kc, ks, ks, i32, i32.view(-1, 1), 0.1, None, None) is None
-    assert f.prefill(q, kc, kc, ks, ks, i32, None, None, 0, 2, 0.1) is None
+    assert f.prefill(q, kc, kc, ks, ks, i32, None, None, 0, 2, 0, 0.1) is None
     assert f.fresh(q, k, k, i32, i32, 2, 0.1) is None
     cos = torch.ones(4, 128, dtype=torch.float16)
     assert f.prologue(i32.long(), q, k, k, None, None, 1e-6, cos, cos, kc, kc, ks, ks, i32,

@@ -171,7 +171,7 @@ def test_a_failed_launch_raises_and_is_not_tried_again():
 
     address = ctypes.cast(stub, ctypes.c_void_p).value
     entries = ("mskv_store_fp8_kvcache_strided", "mskv_fp8_decode_attention",
-               "mskv_fp8_prefill_attention_ws", "mskv_prefill_attention_strided",
+               "mskv_fp8_prefill_attention_bounded", "mskv_prefill_attention_strided",
                "mskv_qk_norm_rope_store")
     qc = q.contiguous()
     lens = torch.ones(5, dtype=torch.int32, device=H.DEV)

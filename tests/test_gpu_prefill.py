@@ -21,7 +21,7 @@ sys.path.insert(0, GOLDEN)
 import cases  # noqa: E402
 
 from microserve_amd import (  # noqa: E402
-    fp8_chunk_prefill_attention, fp8_varlen_prefill_attention, store_fp8_kvcache)
+    _lib, fp8_chunk_prefill_attention, fp8_varlen_prefill_attention, store_fp8_kvcache)
 
 
 def test_chunk_prefill_reference_case():
@@ -319,3 +319,38 @@ def test_prefill_split_keeps_a_nan_key(at, dtype):
     sees = cached + torch.arange(new) >= at
     nan = torch.isnan(out.float().cpu())
     assert torch.equal(nan.all(-1).all(-1), sees) and torch.equal(nan.any(-1).any(-1), sees)
+
+
+@pytest.mark.parametrize("bound", [None, 1, 203, 700, 3064, 16384, 1 << 40])
+def test_prefill_bound_of_the_keys_changes_no_result(bound):
+    """max_seqlen_k chooses the number of key ranges only: below, at and above
+    the real counts every row matches the oracle."""
+    lq, lk = [40, 74, 1, 64], [40 + 300, 74 + 129, 1 + 2100, 64 + 3000]
+    query, tables, caches, cu_q, cu_k = _varlen_setup(311, lq, lk, 32, 8)
+    tables = torch.nn.functional.pad(tables, (0, 64 - tables.shape[1]), value=-1)
+    scale = H.D ** -0.5
+    out = fp8_varlen_prefill_attention(query.to(H.DEV), *caches, tables.to(H.DEV),
+                                       cu_q.to(H.DEV), cu_k.to(H.DEV), max(lq), scale,
+                                       max_seqlen_k=bound)
+    torch.cuda.synchronize()
+    kc, vc, ks, vs = H.cache_to_numpy(*caches)
+    H.assert_attention_close(out, O.varlen_prefill_attention(query, kc, vc, ks, vs, tables, cu_q,
+                                                             cu_k, scale))
+
+
+def test_short_chunk_under_a_wide_table_runs_unsplit():
+    """The host knows a chunk's keys: under any table it gives the bits of the
+    entry that never splits."""
+    new, cached = 40, 300
+    query, tables, caches, _, _ = _varlen_setup(321, [new], [new + cached], 32, 8)
+    tables = torch.nn.functional.pad(tables, (0, 64 - tables.shape[1]), value=-1).to(H.DEV)
+    q = query.to(H.DEV)
+    got = fp8_chunk_prefill_attention(q, *caches, tables, cached, 0.088)
+    want = torch.empty_like(q)
+    lib = _lib.load()
+    assert lib.mskv_fp8_prefill_attention(
+        q.data_ptr(), *[c.data_ptr() for c in caches], tables.data_ptr(), None, None, cached,
+        want.data_ptr(), 1, new, new, 32, 8, H.D, H.BLOCK, caches[0].shape[0], 64, 0.088,
+        _lib.act_dtype(q), _lib.stream_of(q)) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
