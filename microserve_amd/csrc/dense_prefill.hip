@@ -77,6 +77,7 @@ struct DenseArgs {
   int64_t k_stride, v_stride;  // elements between the tokens of key / value
   int hq, hk, group, gc, qgroups, tpr;
   float scale_log2;
+  int turn;  // whether the sequences change places from query block to query block
 };
 
 // LDS byte offset of 16-byte chunk `chunk` (0..15) of tile row `row`
@@ -110,7 +111,16 @@ __global__ __launch_bounds__(kDThreads, 2) void dense_prefill_kernel(DenseArgs a
   // dispatched before any shorter ones (longest-first across the whole
   // grid, not within each sequence); measured 3.8% faster than query
   // blocks varying fastest
-  const int s = blockIdx.y;
+  // A ragged batch leaves most of the grid without rows, and the rows of one
+  // long sequence in every (sequences x units)-th workgroup.  Workgroups go
+  // to XCDs and CUs in turn, so a stride that is a multiple of a power of two
+  // piles them on a fraction of the chip: the small grids of an even number
+  // of sequences move them by a scrambled amount for each query block.
+  // (Moved by one per block, counts of 2^n + 1 pile up instead; an odd count
+  // needs no move, and would be 4 to 11% slower with it.)
+  int s = blockIdx.y;
+  if (kDBlocks == 1 && a.turn)
+    s = (int)((blockIdx.y + (blockIdx.z * 2654435761u >> 16)) % gridDim.y);
   const int unit = blockIdx.x;
   const int kvh = unit / a.qgroups;
   const int qgi = unit - kvh * a.qgroups;
@@ -375,7 +385,7 @@ static hipError_t launch_dense(const DenseArgs& a, int num_seqs, int max_seqlen_
   return hipGetLastError();
 }
 
-// Below this many workgroups of one-block waves, one block per wave.  Two
+// Up to this many workgroups of one-block waves, one block per wave.  Two
 // workgroups are resident per CU, 512 on the chip: a grid of about two
 // rounds is bound by its longest workgroup's chain of tiles, and a tile of
 // one block takes 1.1 us against 1.8 us for three.  Larger grids are bound by
@@ -386,21 +396,37 @@ static hipError_t launch_dense(const DenseArgs& a, int num_seqs, int max_seqlen_
 //   (1256), 3000 103.1 / 105.5 (1504); 3 x 1000 43.9 / 45.8 (1512);
 //   64 q heads 1000 39.8 / 30.6 (1000), 2000 80.4 / 90.5 (2000);
 //   40 q heads 2000 71.0 / 63.2 (1336); 16 q heads 4000 117.8 / 83.5 (1000).
+// Where every sequence is a single tile there is no chain to shorten: three
+// blocks stay ahead if their grid is at most one workgroup per CU (24 x 33
+// tokens 8.0 / 8.3, three blocks' workgroups 192) or just fills the chip (32
+// x 64 13.1 / 14.4, 512); in between one block is faster (24 x 64 11.8 /
+// 10.0, 384), as it is where both grids have the same workgroups (32 q / 32
+// kv heads, 24 x 33 11.4 / 7.7).
+// A ragged batch's grid (every sequence has the longest one's query blocks)
+// may be far larger than the workgroups that have rows, which decide as long
+// as they are spread over the chip (`turn`): 32/8, one of 1000 tokens and 3
+// of 50 36 / 27, one of 1800 and 15 of 30 95 / 47; 8 q / 1 kv heads, one of
+// 1500 and 31 of 20 127 / 38.  (Without the turn these were 46, 129, 176.)
 constexpr int64_t kDSmallGrid = 1280;
 
 template <typename T>
-static hipError_t launch_dense_sized(const DenseArgs& a, int num_seqs, int max_seqlen_q,
-                                     hipStream_t st) {
-  // workgroups with rows: no more than the grid holds, and no more than the
-  // tokens fill plus one partial block per sequence
-  const int64_t tok = kDWaves * a.tpr;
-  const int64_t blocks =
-      min((int64_t)num_seqs * ((max_seqlen_q + tok - 1) / tok), a.total_q / tok + num_seqs);
+static hipError_t launch_dense_sized(DenseArgs a, int num_seqs, int max_seqlen_q, hipStream_t st) {
+  const int64_t units = a.hk * a.qgroups, tok = kDWaves * a.tpr;
+  const int64_t per_seq = ((int64_t)max_seqlen_q + tok - 1) / tok;
+  const int64_t one = num_seqs * per_seq * units;
+  const int64_t three = num_seqs * (((int64_t)max_seqlen_q + 3 * tok - 1) / (3 * tok)) * units;
+  // workgroups with rows: no more than the tokens fill plus one partial block
+  // per sequence
+  const int64_t filled = std::min(one, (a.total_q / tok + num_seqs) * units);
+  const bool single = max_seqlen_q <= kDStep;  // one tile per sequence
+  const bool small = one > kDSmallGrid ? filled <= kDSmallGrid && !single
+                     : single          ? one <= 512 || one == three || (three > 256 && three < 512)
+                                       : true;
+  a.turn = one > kDSmallGrid && num_seqs % 2 == 0;
   // the one-block grid's z must fit its limit too (max_seqlen_q may be far
   // above the tokens there are)
-  const bool one = blocks * a.hk * a.qgroups <= kDSmallGrid && (max_seqlen_q + tok - 1) / tok <= 65535;
-  return one ? launch_dense<T, 1>(a, num_seqs, max_seqlen_q, st)
-             : launch_dense<T, 3>(a, num_seqs, max_seqlen_q, st);
+  return small && per_seq <= 65535 ? launch_dense<T, 1>(a, num_seqs, max_seqlen_q, st)
+                                   : launch_dense<T, 3>(a, num_seqs, max_seqlen_q, st);
 }
 
 }  // namespace mskv

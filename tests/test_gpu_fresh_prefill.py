@@ -137,9 +137,18 @@ def test_fresh_prefill_random_shapes(case):
     # 12 (group 5), 4 (group 16); tiles of 64 keys
     (32, 8, [15, 16, 17, 1, 63, 64, 65, 128, 129]), (40, 8, [11, 12, 13, 65]),
     (16, 1, [3, 4, 5, 64]),
-    # the last length below and the first above the small grid's limit: 1280
-    # workgroups of 16 tokens and 8 heads, and one more
-    (32, 8, [2544]), (32, 8, [2561]),
+    # the last length of the small grid and the first above it: 1280
+    # workgroups of 16 tokens and 8 heads, and 1288
+    (32, 8, [2560]), (32, 8, [2561]),
+    # ragged batches, whose grid is larger than that but mostly without rows:
+    # an even count of sequences (moved about from block to block), an odd
+    # one, one past the limit of workgroups with rows
+    (32, 8, [40] * 3 + [1000]), (32, 8, [7, 900] + [1] * 14), (16, 1, [8] * 31 + [300]),
+    (32, 8, [40] * 4 + [1000]), (32, 8, [2200, 1, 600]), (8, 8, [1, 2500, 3, 100] * 2),
+    # single tiles: at and above 512 workgroups, both sides of 256 and 512
+    # of the three-block grid
+    (32, 8, [16] * 64), (32, 8, [16] * 65), (32, 8, [33] * 24), (32, 8, [64] * 24),
+    (32, 8, [64] * 32), (32, 8, [17] * 80), (8, 8, [64] * 70),
 ])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_fresh_prefill_block_sizes_at_their_edges(hq, hk, lens, dtype):
