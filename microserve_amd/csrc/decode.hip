@@ -1048,21 +1048,26 @@ extern "C" int mskv_decode_num_splits(int batch, int num_q_heads,
   if (pps < 1) pps = 1;
   if (pps > mskv::kMaxPagesPerSplit) pps = mskv::kMaxPagesPerSplit;
   int64_t splits = (w + pps - 1) / pps;
-  // A page per split leaves half the waves idle: finer splits, of two steps at least,
-  // up to two per wave slot (one is expected to run, see split_tokens_of),
-  // as long as the grid and the partials stay small.  Only where they follow
-  // the lengths: at the shape's own split a page each, more splits than
-  // table entries would start past an int's tokens at the largest pages
-  // (512 splits of 2^23 tokens).
+  // A page per split leaves half the waves idle: finer splits, of two steps at
+  // least, as long as the partials stay small and the grid is one workgroup
+  // per CU: past that, the empty splits of short sequences hold CUs that full
+  // ones wait for.  (Two per CU, tables of pages of 256, bf16 cache, us at a
+  // page per split / one / two workgroups per CU: 64 q / 8 kv heads, 4 x 16 to
+  // 8192 tokens 18.6 / 16.4 / 23.3; 8 q / 1 kv heads, 32 x 2048 12.8 / 12.8 /
+  // 14.7, 64 x 16 to 1536 13.0 / 13.2 / 18.3.)  And only if they are half as
+  // many again: below that their bookkeeping, 0.3 to 0.8 us, is all that
+  // changes (8 q / 1 kv, 6 x 8192: 32 splits 13.4, 42 14.2).
+  // Only where they follow the lengths: at the shape's own split a page each,
+  // more splits than table entries would start past an int's tokens at the
+  // largest pages (512 splits of 2^23 tokens).
   if (splits > 1 && 2 * w * base <= mskv::kTargetWaves && block_size > 0 &&
       (int64_t)w * block_size <= mskv::kFollowMaxTokens) {
     const int64_t per = (base / batch + mskv::kWavesPerWG - 1) / mskv::kWavesPerWG * batch;
-    int64_t fine = 2 * mskv::kTargetWaves / base;
-    fine = std::min(fine, (int64_t)w * block_size / (mskv::kMinSplitSteps * mskv::kStep));
-    fine = std::min(fine, mskv::kWideGridMax / per);
+    int64_t fine = (int64_t)w * block_size / (mskv::kMinSplitSteps * mskv::kStep);
+    fine = std::min(fine, mskv::kWideGridMax / 2 / per);
     fine = std::min(fine, (int64_t)(mskv::kFinePartialBytes /
                                     ((int64_t)batch * num_q_heads * (mskv::kHeadDim + 1) * 4)));
-    splits = std::max(splits, fine);
+    if (2 * fine >= 3 * splits) splits = fine;
   }
   return (int)splits;
 }

@@ -76,6 +76,21 @@ def test_every_split_starts_within_an_int_of_tokens():
                     assert s <= w or w * block <= 1 << 22, (batch, hq, hk, w, block, s)
 
 
+def test_splits_finer_than_a_page_fit_one_workgroup_per_cu():
+    lib = _lib.load()
+    finer = 0
+    for hq, hk in ((32, 8), (64, 8), (16, 8), (8, 1), (4, 2), (24, 1), (32, 32)):
+        units = hk * -(-(hq // hk) // 16)
+        for batch in (1, 2, 3, 6, 8, 12, 16, 32, 64, 70, 100, 300):
+            for w in (1, 2, 3, 4, 6, 16, 32, 64, 128):
+                s = lib.mskv_decode_num_splits(batch, hq, hk, w, 256)
+                if s > w:
+                    finer += 1
+                    assert batch * -(-units // 8) * s <= 256 and 2 * s >= 3 * w
+                    assert batch * hq * s * 129 * 4 <= 16 << 20
+    assert finer > 50
+
+
 def test_prefill_workspace_stays_small():
     """The partials have a row per query row: a query tensor with more rows
     than max_seqlen_q lets the grid cover must not ask for gigabytes."""

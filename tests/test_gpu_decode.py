@@ -541,8 +541,10 @@ def test_decode_concurrent_streams_match_the_oracle():
     (32, 8, [4096, 16, 700], 32),
     # one sequence, splits finer than a page (more of them than table entries)
     (16, 8, [700], 0), (32, 8, [64 * 7 + 1], 0), (64, 8, [3000], 0),
-    # a batch past the wave's 64 lanes; a group above 16; few kv heads
-    (16, 8, [1 + 37 * i % 400 for i in range(70)], 4), (24, 1, [500, 90], 40),
+    # a batch past the wave's 64 lanes (one unit, three splits of two pages);
+    # a group above 16; few kv heads
+    (8, 1, [1 + 37 * i % 512 for i in range(70)], 2),
+    (8, 1, [5] * 64 + [512, 0, 1, 300, 65], 2), (24, 1, [500, 90], 40),
     (32, 2, [1000, 31, 2047], 16),
 ])
 def test_decode_splits_that_follow_the_lengths(hq, hk, lens, width, dtype):
@@ -550,6 +552,9 @@ def test_decode_splits_that_follow_the_lengths(hq, hk, lens, width, dtype):
     query, tables, caches = _setup(641 + len(lens) + hq, lens, hq, hk, nb, dtype)
     if width > tables.shape[1]:
         tables = torch.nn.functional.pad(tables, (0, width - tables.shape[1]), value=-1)
+    # more splits than pages, or more than eight of several pages: these follow
+    w, splits = tables.shape[1], decode_num_splits(len(lens), hq, hk, tables.shape[1], H.BLOCK)
+    assert splits > w or 8 < splits <= w / 2
     _, out = _run_and_check(query, lens, tables, caches)
     assert all(torch.all(out[i].float() == 0) for i, n in enumerate(lens) if n == 0)
 
