@@ -125,15 +125,17 @@ struct DecodeArgs {
   uint16_t* out;
   float* part_o;
   float* part_lse;
-  // Work items longest-first (grids of many rounds, else null): item i is
-  // (sequence, split, length, block id of the split's first page), for
-  // the valid splits of the sequences in order of decreasing length, and
-  // rule.info[0] of them are valid.
-  const int4* items;
-  int batch, hq, hk, group, qgroups, bs, w, splits, pages_per_split;
-  SplitRule rule;
+  // what every wave needs before its first K/V load lies in the first 128
+  // bytes (behind `rule`, these cost two more serial reads of the arguments:
+  // 0.5 us of 22 on grids of two short rounds)
   int64_t num_blocks;
   float scale_log2;
+  int batch, hq, hk, group, qgroups, bs, w, splits, pages_per_split;
+  // Work items (grids of many rounds, else null): item i is (sequence, split,
+  // length, block id of the split's first page), the full splits first, then
+  // the sequences' last ones by length; rule.info[0] of them are valid.
+  const int4* items;
+  SplitRule rule;
 };
 
 // Sum / max over the wave with DPP row shifts and the two cross-row swaps
@@ -376,17 +378,16 @@ __device__ __forceinline__ void attend_range(const DecodeArgs& a, int b, int kvh
     const f32x4 vsc0 = *reinterpret_cast<const f32x4*>(sc + 32 + 4 * g);
     const f32x4 vsc1 = *reinterpret_cast<const f32x4*>(sc + 48 + 4 * g);
     float x[8];
-    if (valid == kStep) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      x[r] = s0[r] * ksc0[r];
+      x[4 + r] = s1[r] * ksc1[r];
+    }
+    if (valid != kStep) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        x[r] = s0[r] * ksc0[r];
-        x[4 + r] = s1[r] * ksc1[r];
-      }
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        x[r] = (4 * g + r < valid) ? s0[r] * ksc0[r] : -INFINITY;
-        x[4 + r] = (16 + 4 * g + r < valid) ? s1[r] * ksc1[r] : -INFINITY;
+        if (!(4 * g + r < valid)) x[r] = -INFINITY;
+        if (!(16 + 4 * g + r < valid)) x[4 + r] = -INFINITY;
       }
     }
     float tmax = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])),
@@ -496,84 +497,87 @@ void decode_fp8_kernel(DecodeArgs a) {
   const int lane = threadIdx.x & 63;
   const int g = lane >> 4, n = lane & 15;
   const int unit = blockIdx.x * W + wave;
-  const bool unit_ok = unit < a.hk * a.qgroups;
-  const int kvh = unit / a.qgroups;
-  const int hig = (unit - kvh * a.qgroups) * 16 + n;  // head within its group
-  const bool head_ok = hig < a.group;
-  const int qh = kvh * a.group + hig;
-
-  // one split of one sequence; blk_first: the block id of its first page
-  auto run = [&](int b, int split, int len_raw, int blk_first, int split_tokens) {
-    const int t_begin = split * split_tokens;
-    // tokens past the block table's width are not addressable: ignore them
-    const int L = min(len_raw, a.w * a.bs);
-    if (L <= 0) {
-      if (a.splits == 1 && split == 0 && head_ok) {
-        uint16_t* op = a.out + ((int64_t)b * a.hq + qh) * kHeadDim;
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt)
-          *reinterpret_cast<u32x2*>(op + 16 * dt + 4 * g) = u32x2{0u, 0u};
-      }
-      return;
-    }
-    if (t_begin >= L) return;
-    const int t_end = min(L, t_begin + split_tokens);
-    if (kMode == kFollow && split_tokens != a.rule.fixed)
-      blk_first = __builtin_amdgcn_readfirstlane(a.bt[(int64_t)b * a.w + t_begin / a.bs]);
-
-    f32x4 acc[8];
-    float m, l;
-    attend_range<T>(a, b, kvh, qh, head_ok, t_begin, t_end, blk_first, lane, kv_lds_all[wave],
-                    s_lds_all[wave], acc, m, l);
-
-    // splits that hold tokens of this sequence; a sequence that fits in one
-    // split is written here directly
-    const int nvalid = min(a.splits, (L + split_tokens - 1) / split_tokens);
-    if (!head_ok) return;
-    if (nvalid == 1) {
-      write_output<T>(a.out + ((int64_t)b * a.hq + qh) * kHeadDim, acc, l, g);
-      return;
-    }
-    // this split's partial, merged by a combine kernel
-    const int64_t row = ((int64_t)b * a.hq + qh) * a.splits + split;
-    write_partial(a.part_o + row * kHeadDim, a.part_lse + row, acc, m, l, g);
-  };
-
+  // The sequence, its length and the split's first block id are read
+  // together, first thing, so the first K/V loads wait for one memory round
+  // trip, not a chain of them (readfirstlane is convergent, so the compiler
+  // cannot sink a read below the branches that use it).
+  int b, split, len_raw, blk_first, split_tokens;
   if constexpr (kMode == kItems) {
     const int item = blockIdx.z * a.splits + blockIdx.y;
     const int4 e = a.items[item];
     const int count = __builtin_amdgcn_readfirstlane(a.rule.info[0]);
-    const int split_tokens = __builtin_amdgcn_readfirstlane(a.rule.info[1]);
-    const int b = __builtin_amdgcn_readfirstlane(e.x);
-    const int split = __builtin_amdgcn_readfirstlane(e.y);
-    const int len_raw = __builtin_amdgcn_readfirstlane(e.z);
-    const int blk_first = __builtin_amdgcn_readfirstlane(e.w);
-    if (item >= count || !unit_ok) return;
+    split_tokens = __builtin_amdgcn_readfirstlane(a.rule.info[1]);
+    b = __builtin_amdgcn_readfirstlane(e.x);
+    split = __builtin_amdgcn_readfirstlane(e.y);
+    len_raw = __builtin_amdgcn_readfirstlane(e.z);
+    blk_first = __builtin_amdgcn_readfirstlane(e.w);
+    if (item >= count) return;
     if ((unsigned)b >= (unsigned)a.batch || (unsigned)split >= (unsigned)a.splits) return;
-    run(b, split, len_raw, blk_first, split_tokens);
-  } else {
-    // The sequence, its length and the split's first block id are read
-    // together, first thing, so the first K/V loads wait for one memory
-    // round trip, not a chain of them (readfirstlane is convergent, so the
-    // compiler cannot sink a read below the branches that use it).  The
-    // split's first page, clamped to the table (splits finer than a page may
-    // be more than its entries), is that of the shape's own split; another
-    // one is read later.  Splits that follow the lengths put the empty ones
-    // last by taking z as the split (in between, every 2 us wave of them
-    // delays the valid ones behind: batch 16 x 4096 tokens, half of 32
-    // splits empty, 43 against 29 us); the sequences rotate with it, so that
-    // one sequence's splits spread over the XCDs.
-    constexpr bool kAdapt = kMode == kFollow;
-    const int own = kAdapt ? lane_length(a.seqlens, a.rule) : 0;
-    const int split = kAdapt ? blockIdx.z : blockIdx.y;
-    const int b = kAdapt ? (blockIdx.y + blockIdx.z) % a.batch : blockIdx.z;
-    const int len_raw = __builtin_amdgcn_readfirstlane(a.seqlens[b]);
-    const int blk_first = __builtin_amdgcn_readfirstlane(
+  } else if constexpr (kMode == kFollow) {
+    // The block id is that of the shape's own split, clamped to the table
+    // (splits finer than a page may be more than its entries); another one is
+    // read later.  The empty splits come last by taking z as the split (in
+    // between, every 2 us wave of them delays the valid ones behind: batch 16
+    // x 4096 tokens, half of 32 splits empty, 43 against 29 us); the
+    // sequences rotate with it, so that one sequence's splits spread over the
+    // XCDs.
+    const int own = lane_length(a.seqlens, a.rule);
+    split = blockIdx.z;
+    b = (blockIdx.y + blockIdx.z) % a.batch;
+    len_raw = __builtin_amdgcn_readfirstlane(a.seqlens[b]);
+    blk_first = __builtin_amdgcn_readfirstlane(
         a.bt[(int64_t)b * a.w + min(split * a.pages_per_split, a.w - 1)]);
-    if (!unit_ok) return;
-    run(b, split, len_raw, blk_first,
-        kAdapt ? split_tokens_of(own, len_raw, a.seqlens, a.rule) : a.rule.fixed);
+    if (unit >= a.hk * a.qgroups) return;
+    split_tokens = split_tokens_of(own, len_raw, a.seqlens, a.rule);
+  } else {
+    // (the split's first page is inside the table: split * pages_per_split <
+    // w for every split count of these shapes)
+    split = blockIdx.y;
+    b = blockIdx.z;
+    len_raw = __builtin_amdgcn_readfirstlane(a.seqlens[b]);
+    blk_first =
+        __builtin_amdgcn_readfirstlane(a.bt[(int64_t)b * a.w + split * a.pages_per_split]);
+    split_tokens = a.pages_per_split * a.bs;
   }
+  if (unit >= a.hk * a.qgroups) return;
+  const int kvh = unit / a.qgroups;
+  const int hig = (unit - kvh * a.qgroups) * 16 + n;  // head within its group
+  const bool head_ok = hig < a.group;
+  const int qh = kvh * a.group + hig;
+  const int t_begin = split * split_tokens;
+  // tokens past the block table's width are not addressable: ignore them
+  const int L = min(len_raw, a.w * a.bs);
+
+  if (L <= 0) {
+    if (a.splits == 1 && split == 0 && head_ok) {
+      uint16_t* op = a.out + ((int64_t)b * a.hq + qh) * kHeadDim;
+#pragma unroll
+      for (int dt = 0; dt < 8; ++dt)
+        *reinterpret_cast<u32x2*>(op + 16 * dt + 4 * g) = u32x2{0u, 0u};
+    }
+    return;
+  }
+  if (t_begin >= L) return;
+  const int t_end = min(L, t_begin + split_tokens);
+  if (kMode == kFollow && split_tokens != a.rule.fixed)
+    blk_first = __builtin_amdgcn_readfirstlane(a.bt[(int64_t)b * a.w + t_begin / a.bs]);
+
+  f32x4 acc[8];
+  float m, l;
+  attend_range<T>(a, b, kvh, qh, head_ok, t_begin, t_end, blk_first, lane, kv_lds_all[wave],
+                  s_lds_all[wave], acc, m, l);
+
+  // splits that hold tokens of this sequence; a sequence that fits in one
+  // split is written here directly
+  const int nvalid = min(a.splits, (L + split_tokens - 1) / split_tokens);
+  if (!head_ok) return;
+  if (nvalid == 1) {
+    write_output<T>(a.out + ((int64_t)b * a.hq + qh) * kHeadDim, acc, l, g);
+    return;
+  }
+  // this split's partial, merged by a combine kernel
+  const int64_t row = ((int64_t)b * a.hq + qh) * a.splits + split;
+  write_partial(a.part_o + row * kHeadDim, a.part_lse + row, acc, m, l, g);
 }
 
 // A merge state over some splits of one row, held in plain registers: the
@@ -862,7 +866,7 @@ constexpr int kOrderMaxBatch = 4096;
 
 __global__ __launch_bounds__(kOrderThreads) void decode_order_kernel(
     const int32_t* __restrict__ seqlens, const int32_t* __restrict__ bt, int4* __restrict__ items,
-    int bs, int w, SplitRule rule) {
+    int bs, int w, int pages_per_split, SplitRule rule) {
   constexpr int kWaves = kOrderThreads / 64;
   __shared__ int s_steps[kWaves], s_long[kWaves], s_off[kWaves], s_tot[kWaves], s_part[kWaves];
   const int b = blockIdx.x;
@@ -870,7 +874,7 @@ __global__ __launch_bounds__(kOrderThreads) void decode_order_kernel(
   const int len_b = seqlens[b];
   // this thread's first split's block id under the shape's own split, read
   // with the lengths
-  const int fixed_page = tid * (rule.fixed / bs);
+  const int fixed_page = tid * pages_per_split;
   const int blk_fixed = tid < rule.splits && fixed_page < w ? bt[(int64_t)b * w + fixed_page] : 0;
   int split_tokens = rule.fixed;
   if (rule.adapt) {
@@ -984,7 +988,8 @@ static hipError_t launch_decode(const DecodeArgs& a, int batch, hipStream_t stre
     const dim3 grid((unsigned)((units + per_wg - 1) / per_wg), (unsigned)a.splits,
                     (unsigned)batch);
     hipLaunchKernelGGL(decode_order_kernel, dim3((unsigned)batch), dim3(kOrderThreads), 0, stream,
-                       a.seqlens, a.bt, const_cast<int4*>(a.items), a.bs, a.w, a.rule);
+                       a.seqlens, a.bt, const_cast<int4*>(a.items), a.bs, a.w, a.pages_per_split,
+                       a.rule);
     const hipError_t eo = hipGetLastError();
     if (eo != hipSuccess) return eo;
     if (wide)
