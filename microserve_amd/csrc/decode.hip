@@ -106,6 +106,7 @@ struct SplitRule {
   int fixed;       // split_tokens from the shapes: a whole number of pages
   int max_tokens;  // addressable tokens of a sequence (the table's width)
   bool adapt;      // split_tokens follows the lengths, else it is `fixed`
+  int min_gain;    // steps that splitting must save where `fixed` would not split
   // 1 / the splits that run at once (CUs over workgroups per split, less
   // half a split per sequence), and 1 / splits
   float inv_slots, inv_splits;
@@ -164,13 +165,14 @@ __device__ __forceinline__ int wave_max_u31(int v) {  // of values >= 0
 __device__ __forceinline__ int steps_of_length(int len, const SplitRule& r) {
   return (max(0, min(len, r.max_tokens)) + kStep - 1) / kStep;
 }
-// (longest / splits is at least 1 / longest away from a whole number or on
-// it, 2^-17 with max_tokens <= 2^22, so the float product never rounds it
-// down past one)
+// (Where longest / splits is not whole, it lies at least 1 / splits above the
+// whole number q below it; q * splits <= longest <= 2^17 with max_tokens <=
+// 2^22, so the float product's error, q * 2^-23, never rounds it down to q.)
 __device__ __forceinline__ int split_tokens_from(int steps, int longest, const SplitRule& r) {
   const int per = max((int)ceilf(fmaxf((float)steps * r.inv_slots, (float)longest * r.inv_splits)),
                       kMinSplitSteps);
-  return min(per * kStep, r.fixed);
+  const bool whole = longest * kStep <= r.fixed && longest - per < r.min_gain;
+  return min((whole ? max(longest, per) : per) * kStep, r.fixed);
 }
 
 // The tokens per split of this step, from the lengths on the device: a
@@ -181,6 +183,14 @@ __device__ __forceinline__ int split_tokens_from(int steps, int longest, const S
 // split per sequence for its ragged end); a split has two steps at least,
 // the longest sequence fits in the splits there are, and the shape's own
 // split, which fills the chip when every sequence is full, is the most.
+// With work items, where that would not split any sequence, splitting costs
+// partials and a merge of every row, about a step's time per 1000 rows, and
+// has to shorten the longest chain by more (min_gain; 128 sequences of 100
+// tokens, 8192 rows under 128-entry tables: 16.0 us whole, 22.8 as splits of
+// three steps).  (The smaller grids' merges cost less: 32 x 128, 2048 rows,
+// 12.4 whole, 10.8 in splits of two steps.)  Contexts that end within their
+// first split pay for reading the lengths: 1 to 64 of 64 tokens under tables
+// of several pages 0.5 to 0.8 us of 6 to 9.
 // Whole steps, not whole pages.  With work items the pre-pass applies the
 // rule and leaves its result in rule.info.  Measured against the shape's split, us:
 // batch 16, 64 to 4096 tokens under 128-entry tables 77 -> 23 (the layer's
@@ -559,7 +569,7 @@ void decode_fp8_kernel(DecodeArgs a) {
   }
   if (t_begin >= L) return;
   const int t_end = min(L, t_begin + split_tokens);
-  if (kMode == kFollow && split_tokens != a.rule.fixed)
+  if (kMode == kFollow && split > 0 && split_tokens != a.rule.fixed)
     blk_first = __builtin_amdgcn_readfirstlane(a.bt[(int64_t)b * a.w + t_begin / a.bs]);
 
   f32x4 acc[8];
@@ -872,14 +882,16 @@ __global__ __launch_bounds__(kOrderThreads) void decode_order_kernel(
   const int b = blockIdx.x;
   const int tid = threadIdx.x;
   const int len_b = seqlens[b];
+  // this thread's first length, read once for both passes
+  const int len_own = tid < rule.batch ? seqlens[tid] : 0;
   // this thread's first split's block id under the shape's own split, read
   // with the lengths
   const int fixed_page = tid * pages_per_split;
   const int blk_fixed = tid < rule.splits && fixed_page < w ? bt[(int64_t)b * w + fixed_page] : 0;
   int split_tokens = rule.fixed;
   if (rule.adapt) {
-    int steps = 0, longest = 0;
-    for (int j = tid; j < rule.batch; j += kOrderThreads) {
+    int steps = steps_of_length(len_own, rule), longest = steps;
+    for (int j = tid + kOrderThreads; j < rule.batch; j += kOrderThreads) {
       const int n = steps_of_length(seqlens[j], rule);
       steps += n;
       longest = max(longest, n);
@@ -907,7 +919,7 @@ __global__ __launch_bounds__(kOrderThreads) void decode_order_kernel(
   const int rest_b = key - full_b * split_tokens;
   int off = 0, tot = 0, ahead = 0, parts = 0;
   for (int j = tid; j < rule.batch; j += kOrderThreads) {
-    const int kj = max(0, min(seqlens[j], rule.max_tokens));
+    const int kj = max(0, min(j == tid ? len_own : seqlens[j], rule.max_tokens));
     const int full = kj / split_tokens, rest = kj - full * split_tokens;
     off += j < b ? full : 0;
     tot += full;
@@ -935,10 +947,10 @@ __global__ __launch_bounds__(kOrderThreads) void decode_order_kernel(
   if (b == 0 && tid < 2) rule.info[tid] = tid == 0 ? count : split_tokens;
   const int nv_b = full_b + (rest_b > 0);
   for (int sp = tid; sp < nv_b; sp += kOrderThreads) {
-    // (a split with tokens starts inside the table)
+    // (a split with tokens starts inside the table, whose tokens fit an int)
     const int blk = sp == tid && split_tokens == rule.fixed
                         ? blk_fixed
-                        : bt[(int64_t)b * w + (int64_t)sp * split_tokens / bs];
+                        : bt[(int64_t)b * w + (uint32_t)(sp * split_tokens) / (uint32_t)bs];
     items[sp < full_b ? first + sp : fulls + (part & 0xFFFF)] = int4{b, sp, len_b, blk};
   }
 }
@@ -1162,17 +1174,25 @@ static int decode_checked(const void* query, const void* k_cache, const void* v_
   const int64_t per_split = (num_kv_heads * a.qgroups + kWavesPerWG - 1) / kWavesPerWG;
   const int64_t slots =
       std::max<int64_t>(256 / per_split - batch / 2, std::max<int64_t>(128 / per_split, 1));
-  // (A page per split is short enough as it is, and up to eight splits are
-  // the shapes whose tables fit the lengths: 64 x 4096 tokens would pay 0.5
-  // us for the same splits.)
+  // (Shapes of one page per split, and of up to eight splits, keep the layout
+  // of the shapes.  It is at its best where the lengths fill the tables: 64 x
+  // 4096 tokens would pay 0.5 us to follow the lengths to the same splits.
+  // Lengths well below such tables are served no better for that.)
   const bool fine = num_splits > max_blocks_per_seq;
   const bool adapt = (fine || (a.pages_per_split > 1 && num_splits > 8)) &&
                      (a.items || (batch <= 256 &&
                                   per_split * num_splits * batch <= kWideGridMax)) &&
                      (int64_t)max_blocks_per_seq * block_size <= kFollowMaxTokens;
-  a.rule = SplitRule{batch, num_splits, a.pages_per_split * block_size,
-                     max_blocks_per_seq * block_size, adapt, 1.0f / (float)slots,
-                     1.0f / (float)num_splits, info};
+  const int min_gain = a.items ? 1 + (int)((int64_t)batch * num_q_heads / 1000) : 1;
+  a.rule = SplitRule{batch,
+                     num_splits,
+                     a.pages_per_split * block_size,
+                     max_blocks_per_seq * block_size,
+                     adapt,
+                     min_gain,
+                     1.0f / (float)slots,
+                     1.0f / (float)num_splits,
+                     info};
   a.num_blocks = num_blocks;
   a.scale_log2 = softmax_scale * kLog2e;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
