@@ -375,7 +375,15 @@ __global__ __launch_bounds__(kNrThreads) void qk_norm_rope_store_kernel(NormRope
 // us): 16 tokens 8.7 / 6.2, 256 9.1 / 6.5, 1000 12.0 / 9.3 (1500 workgroups),
 // 2000 14.8 / 14.6 (3000), 4000 24.0 / 25.1; 64 q heads, fp16, 1000 tokens
 // 13.8 / 12.5 (2500).  A row's arithmetic is the same in both.
+// Fewer than 32 heads per token (few kv heads per rank) mean more tokens, whose
+// rotary rows every single row reads again, so the line lies lower: 8 q / 1 kv
+// heads 5760 tokens (1800) 9.2 / 8.4, 6720 (2100) 9.0 / 9.1, 8192 (2560) 9.5 /
+// 10.7; 16 q / 1 3200 (1800) 8.3 / 8.0, 3733 (2100) 7.7 / 8.3; 4 q / 2 6000
+// (1500) 8.1 / 7.1, 7200 (1800) 7.9 / 8.1; 8 q / 2 4800 (1800) 8.0 / 8.0, 6826
+// (2560) 9.3 / 10.5.
 constexpr int64_t kNrSmallBlocks = 2560;
+constexpr int64_t kNrSmallBlocksFewHeads = 1700;
+constexpr int kNrFewHeads = 32;
 
 template <typename T, int kNrChunk>
 static hipError_t launch_chunks(NormRopeArgs a, int64_t num_tokens, int slot_dtype,
@@ -398,7 +406,8 @@ static hipError_t launch_chunks(NormRopeArgs a, int64_t num_tokens, int slot_dty
 template <typename T>
 static hipError_t launch_norm_rope(const NormRopeArgs& a, int64_t num_tokens, int slot_dtype,
                                    hipStream_t stream) {
-  return a.rows <= kNrSmallBlocks * kNrGroups
+  const int64_t small = a.heads < kNrFewHeads ? kNrSmallBlocksFewHeads : kNrSmallBlocks;
+  return a.rows <= small * kNrGroups
              ? launch_chunks<T, 1>(a, num_tokens, slot_dtype, stream)
              : launch_chunks<T, 4>(a, num_tokens, slot_dtype, stream);
 }

@@ -244,14 +244,14 @@ def test_attention_forward_fused_equals_unfused(mode):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("hq,hk", [(32, 8), (5, 3)])
-def test_one_row_and_four_row_chunks_agree(hq, hk, dtype):
-    """A call past the small grid's limit (2560 workgroups of 32 rows) takes
-    four rows per lane group; the same tokens in two calls below it take one.
+@pytest.mark.parametrize("hq,hk,limit", [(32, 8, 2560), (5, 3, 2560), (5, 3, 1700)])
+def test_one_row_and_four_row_chunks_agree(hq, hk, limit, dtype):
+    """A call past the small grid's limit (2560 workgroups of 32 rows, 1700 with
+    fewer than 32 heads a token) takes four rows per lane group; the same tokens in two calls below it take one.
     Outputs, cache bytes and scales are the same bits, head counts that are
     not multiples of four included."""
     from tests import gpu_helpers as H
-    n = 2560 * 32 // (hq + 2 * hk) + 1
+    n = limit * 32 // (hq + 2 * hk) + 1
     gen = torch.Generator(device=H.DEV).manual_seed(911)
     qkv = torch.randn(n, (hq + 2 * hk) * H.D, generator=gen, device=H.DEV).to(dtype)
     q, k, v = (t.view(n, -1, H.D) for t in
