@@ -198,6 +198,42 @@ def test_prefills_reject_pointers_off_16_bytes():
             assert fresh(**{name: by}) == EINVAL
 
 
+def test_strided_and_workspace_entries_validate_without_launch():
+    lib = _lib.load()
+    EINVAL, EUNSUP, EWS, A = -1, -2, -3, 1 << 20
+    row = 8 * 128
+
+    def store(ks=row, vs=row, act=1):
+        return lib.mskv_store_fp8_kvcache_strided(A, ks, A, vs, A, A, A, A, A, 1, 4, 8, 128, 100,
+                                                  act, None)
+
+    def fresh(ks=row, vs=row, num_seqs=1):
+        return lib.mskv_prefill_attention_strided(A, A, ks, A, vs, A, A, A, num_seqs, 10, 10, 10,
+                                                  32, 8, 128, 0.1, 1, None)
+
+    for call in (store, fresh):
+        for bad in (row - 8, 0, -row, row + 4, row + 1):  # below a row, off 16 bytes
+            assert call(ks=bad) == EINVAL and call(vs=bad) == EINVAL
+    assert store(ks=row + 2, act=_lib.FLOAT32) == EINVAL   # fp32: 16 bytes are 4 elements
+    assert store(ks=row - 4, act=_lib.FLOAT32) == EINVAL
+    # 64 rows of a tile must stay within 32-bit offsets
+    assert fresh(ks=1 << 24) == EUNSUP and fresh(vs=(1 << 24) + 8) == EUNSUP
+    assert fresh(num_seqs=0) == 0 and fresh(ks=row + 4, num_seqs=0) == EINVAL
+
+    def paged(ws=A, n=0, keys=0):
+        return lib.mskv_fp8_prefill_attention_bounded(
+            A, A, A, A, A, A, None, None, 3000, A, 1, 64, 64, keys, 32, 8, 128, 256, 100, 12, 0.1,
+            1, ws, n, None)
+
+    need = lib.mskv_fp8_prefill_bounded_workspace_bytes(1, 64, 64, 3064, 32, 8, 128, 256, 12)
+    assert need > 0
+    for n in (0, 1, need - 1):
+        assert paged(n=n) == EWS and paged(n=n, keys=3064) == EWS
+    assert lib.mskv_fp8_prefill_attention_ws(
+        A, A, A, A, A, A, None, None, 3000, A, 1, 64, 64, 32, 8, 128, 256, 100, 12, 0.1, 1, A,
+        need - 1, None) == EWS
+
+
 def test_wrappers_copy_rows_off_16_bytes():
     import torch
     flat = torch.arange(3 * 4 * 128 + 9).to(torch.bfloat16)

@@ -22,14 +22,34 @@ class _Off:
         return lambda *a: None
 
 
-def _both(monkeypatch, call):
+class _Counted:
+    """The native paths, noting which took a call and which left it."""
+
+    def __init__(self, fast):
+        self.fast, self.took, self.left = fast, [], []
+
+    def __getattr__(self, name):
+        def call(*a):
+            res = getattr(self.fast, name)(*a)
+            (self.left if res is None else self.took).append(name)
+            return res
+        return call
+
+
+def _both(monkeypatch, entry, call):
+    """`call` on the native path, which must take it, and on the wrappers' own:
+    the same bytes (each result copied before the next call)."""
     _lib.load()
-    fast = call()
     with monkeypatch.context() as m:
+        counted = _Counted(_lib.fast)
+        m.setattr(_lib, "fast", counted)
+        fast = call()
+        kept = [None if t is None else t.clone() for t in fast]
+        assert counted.took == [entry] and not counted.left
         m.setattr(_lib, "fast", _Off())
         slow = call()
     torch.cuda.synchronize()
-    for a, b in zip(fast, slow):
+    for a, b in zip(kept, slow):
         assert (a is None and b is None) or torch.equal(a.view(torch.uint8), b.view(torch.uint8))
     return fast
 
@@ -52,23 +72,29 @@ def test_native_paths_give_the_wrappers_results(dtype, monkeypatch):
         store_fp8_kvcache(k.contiguous(), v, *c, slots)
         return c
 
-    caches = _both(monkeypatch, store)
+    caches = _both(monkeypatch, "store", store)
     qc = q.contiguous()
     lens = torch.tensor([300, 1, 0, 256, 40], dtype=torch.int32, device=H.DEV)
     tables = torch.tensor([[0, 1], [2, -1], [-1, -1], [3, -1], [4, 5]], dtype=torch.int32,
                           device=H.DEV)
     out = torch.empty_like(qc)
-    _both(monkeypatch, lambda: [fp8_decode_attention(qc, *caches, lens, tables, 0.1)])
-    (got,) = _both(monkeypatch,
-                   lambda: [fp8_decode_attention(qc, *caches, lens, tables, 0.1, out=out)])
+    _both(monkeypatch, "decode", lambda: [fp8_decode_attention(qc, *caches, lens, tables, 0.1)])
+
+    def into_out():
+        out.fill_(7.0)
+        return [fp8_decode_attention(qc, *caches, lens, tables, 0.1, out=out)]
+
+    (got,) = _both(monkeypatch, "decode", into_out)
     assert got is out
-    _both(monkeypatch, lambda: [fp8_chunk_prefill_attention(qc, *caches, tables[:1], 200, 0.1)])
+    _both(monkeypatch, "prefill", lambda: [
+        fp8_chunk_prefill_attention(qc, *caches, tables[:1], 200, 0.1)])
     cu = torch.tensor([0, 2, n], dtype=torch.int32, device=H.DEV)
     ck = torch.tensor([0, 300, 500], dtype=torch.int32, device=H.DEV)
-    _both(monkeypatch, lambda: [fp8_varlen_prefill_attention(qc, *caches, tables[:2], cu, ck, 3,
-                                                             0.1)])
+    for bound in (None, 300):
+        _both(monkeypatch, "prefill", lambda: [fp8_varlen_prefill_attention(
+            qc, *caches, tables[:2], cu, ck, 3, 0.1, max_seqlen_k=bound)])
     for kk in (k, k.contiguous()):
-        _both(monkeypatch, lambda: [varlen_attention(qc, kk, v, cu, cu, 3)])
+        _both(monkeypatch, "fresh", lambda: [varlen_attention(qc, kk, v, cu, cu, 3)])
     cos, sin = (torch.randn(64, 1, H.D, device=H.DEV).to(dtype) for _ in range(2))
     w = torch.randn(H.D, device=H.DEV).to(dtype)
     pos = torch.arange(n, device=H.DEV)
@@ -78,7 +104,7 @@ def test_native_paths_give_the_wrappers_results(dtype, monkeypatch):
                 c = H.alloc_cache(6, H.BLOCK, 2)
                 return [*qk_norm_rope_store(pos, q, k, v, weight, weight, 1e-6, cos, sin, *c,
                                             slots, return_k=return_k), *c]
-            _both(monkeypatch, prologue)
+            _both(monkeypatch, "prologue", prologue)
 
 
 @pytest.mark.parametrize("by", [1, 2])

@@ -212,6 +212,8 @@ def test_store_reads_strided_tokens_like_their_copies(n, hk, dtype):
         for key, value in ((view, view.contiguous()), (view.contiguous(), view), (view, view)):
             a, b = H.alloc_cache(4, H.BLOCK, hk), H.alloc_cache(4, H.BLOCK, hk)
             store_fp8_kvcache(key, value, *a, slots)
-            store_fp8_kvcache(key.contiguous(), value.contiguous(), *b, slots)
+            # (clone: a single token's view counts as contiguous wherever it starts)
+            packed = [t.clone(memory_format=torch.contiguous_format) for t in (key, value)]
+            store_fp8_kvcache(*packed, *b, slots)
             for x, y in zip(a, b):
                 assert torch.equal(x.view(torch.uint8), y.view(torch.uint8)), name
