@@ -77,7 +77,6 @@ struct DenseArgs {
   int64_t k_stride, v_stride;  // elements between the tokens of key / value
   int hq, hk, group, gc, qgroups, tpr;
   float scale_log2;
-  int turn;  // whether the sequences change places from query block to query block
 };
 
 // LDS byte offset of 16-byte chunk `chunk` (0..15) of tile row `row`
@@ -91,7 +90,8 @@ __device__ __forceinline__ void lds_load16_d(__amdgpu_buffer_rsrc_t r, void* lds
 }
 
 // kDBlocks: 16-row blocks per wave, 3 or (small grids) 1
-template <typename T, int kDBlocks>
+// kTurn: the sequences change places from query block to query block
+template <typename T, int kDBlocks, bool kTurn>
 __global__ __launch_bounds__(kDThreads, 2) void dense_prefill_kernel(DenseArgs a) {
   using A = Act<T>;
   using x8 = typename A::x8;
@@ -119,7 +119,7 @@ __global__ __launch_bounds__(kDThreads, 2) void dense_prefill_kernel(DenseArgs a
   // (Moved by one per block, counts of 2^n + 1 pile up instead; an odd count
   // needs no move, and would be 4 to 11% slower with it.)
   int s = blockIdx.y;
-  if (kDBlocks == 1 && a.turn)
+  if constexpr (kTurn)
     s = (int)((blockIdx.y + (blockIdx.z * 2654435761u >> 16)) % gridDim.y);
   const int unit = blockIdx.x;
   const int kvh = unit / a.qgroups;
@@ -376,12 +376,12 @@ __global__ __launch_bounds__(kDThreads, 2) void dense_prefill_kernel(DenseArgs a
   }
 }
 
-template <typename T, int kDBlocks>
+template <typename T, int kDBlocks, bool kTurn>
 static hipError_t launch_dense(const DenseArgs& a, int num_seqs, int max_seqlen_q, hipStream_t st) {
   const int per_wg = kDWaves * kDBlocks * a.tpr;
   const dim3 grid((unsigned)(a.hk * a.qgroups), (unsigned)num_seqs,
                   (unsigned)(((int64_t)max_seqlen_q + per_wg - 1) / per_wg));
-  hipLaunchKernelGGL((dense_prefill_kernel<T, kDBlocks>), grid, dim3(kDThreads), 0, st, a);
+  hipLaunchKernelGGL((dense_prefill_kernel<T, kDBlocks, kTurn>), grid, dim3(kDThreads), 0, st, a);
   return hipGetLastError();
 }
 
@@ -404,13 +404,13 @@ static hipError_t launch_dense(const DenseArgs& a, int num_seqs, int max_seqlen_
 // kv heads, 24 x 33 11.4 / 7.7).
 // A ragged batch's grid (every sequence has the longest one's query blocks)
 // may be far larger than the workgroups that have rows, which decide as long
-// as they are spread over the chip (`turn`): 32/8, one of 1000 tokens and 3
+// as they are spread over the chip (kTurn): 32/8, one of 1000 tokens and 3
 // of 50 36 / 27, one of 1800 and 15 of 30 95 / 47; 8 q / 1 kv heads, one of
 // 1500 and 31 of 20 127 / 38.  (Without the turn these were 46, 129, 176.)
 constexpr int64_t kDSmallGrid = 1280;
 
 template <typename T>
-static hipError_t launch_dense_sized(DenseArgs a, int num_seqs, int max_seqlen_q, hipStream_t st) {
+static hipError_t launch_dense_sized(const DenseArgs& a, int num_seqs, int max_seqlen_q, hipStream_t st) {
   const int64_t units = a.hk * a.qgroups, tok = kDWaves * a.tpr;
   const int64_t per_seq = ((int64_t)max_seqlen_q + tok - 1) / tok;
   const int64_t one = num_seqs * per_seq * units;
@@ -422,11 +422,12 @@ static hipError_t launch_dense_sized(DenseArgs a, int num_seqs, int max_seqlen_q
   const bool small = one > kDSmallGrid ? filled <= kDSmallGrid && !single
                      : single          ? one <= 512 || one == three || (three > 256 && three < 512)
                                        : true;
-  a.turn = one > kDSmallGrid && num_seqs % 2 == 0;
   // the one-block grid's z must fit its limit too (max_seqlen_q may be far
   // above the tokens there are)
-  return small && per_seq <= 65535 ? launch_dense<T, 1>(a, num_seqs, max_seqlen_q, st)
-                                   : launch_dense<T, 3>(a, num_seqs, max_seqlen_q, st);
+  if (!small || per_seq > 65535) return launch_dense<T, 3, false>(a, num_seqs, max_seqlen_q, st);
+  return one > kDSmallGrid && num_seqs % 2 == 0
+             ? launch_dense<T, 1, true>(a, num_seqs, max_seqlen_q, st)
+             : launch_dense<T, 1, false>(a, num_seqs, max_seqlen_q, st);
 }
 
 }  // namespace mskv
