@@ -88,6 +88,11 @@ int mskv_store_fp8_kvcache_strided(const void* key, int64_t key_stride,
  * Number of split-KV partitions mskv_fp8_decode_attention uses for a shape.
  * Depends on shapes only (never on device sequence lengths), so a captured
  * graph stays valid for any lengths up to max_blocks_per_seq * block_size.
+ * It may exceed max_blocks_per_seq (splits finer than a page).  Which tokens
+ * a split holds may follow the lengths of all sequences in the step (shapes
+ * with more splits than pages, or more than eight splits of several pages):
+ * there the last bits of a sequence's output depend on its neighbours'
+ * lengths, the error does not.
  */
 int mskv_decode_num_splits(int batch, int num_q_heads, int num_kv_heads,
                            int max_blocks_per_seq, int block_size);
@@ -95,7 +100,8 @@ int mskv_decode_num_splits(int batch, int num_q_heads, int num_kv_heads,
 /*
  * Scratch bytes mskv_fp8_decode_attention needs for num_splits (0 if 1):
  * the fp32 split partials and, for shapes of many workgroup rounds, the
- * longest-first work items that a pre-pass kernel writes.
+ * work items (the full splits, then the partial ones by length) that a
+ * pre-pass kernel writes.
  * Contents on entry do not matter.
  */
 size_t mskv_decode_workspace_bytes(int batch, int num_q_heads,
@@ -118,8 +124,8 @@ size_t mskv_decode_workspace_bytes(int batch, int num_q_heads,
  * value mskv_decode_num_splits returns for the shape; when it is above 1 the
  * workspace must hold mskv_decode_workspace_bytes bytes, and a second
  * kernel merges the split partials.
- * Supported: head_dim == 128, block_size % 32 == 0, and a GQA group
- * (num_q_heads / num_kv_heads) of at most 16 or a multiple of 16.
+ * Supported: head_dim == 128, block_size % 32 == 0, num_q_heads a multiple
+ * of num_kv_heads.
  */
 int mskv_fp8_decode_attention(const void* query, const void* k_cache,
                               const void* v_cache, const float* k_scale_cache,

@@ -40,14 +40,15 @@
 //    step i is consumed, so the K/V registers live only while in flight.
 //  * Split-KV: the host picks the split count from shapes only; small grids
 //    choose the tokens per split on the device, from the lengths
-//    (split_tokens_of); each split writes (o / l, m + log2 l) partials and a second kernel merges them:
-//    decode_combine_small_kernel up to 8 splits, decode_combine_kernel up
-//    to 64, decode_combine_wide_kernel beyond (an in-kernel merge needs
+//    (split_tokens_of); each split writes (o / l, m + log2 l) partials and
+//    a second kernel merges them: decode_combine_small_kernel up to 8
+//    splits, decode_combine_kernel up to 64, decode_combine_wide_kernel
+//    beyond (an in-kernel merge needs
 //    agent-scope fences, i.e. an L2 writeback + invalidate per XCD, which
 //    measured 2x slower).  A sequence that fits in one split is written
 //    directly by the split kernel.
 //  * Grids of many rounds (over 512 eight-wave workgroups) run compacted
-//    work items longest-first: a pre-pass on the device lists the valid
+//    work items, the long ones first: a pre-pass on the device lists the valid
 //    splits, full ones first, then the sequences' last ones by length, so
 //    short ones fill the last round and empty splits exit at the end of the
 //    grid.
@@ -192,12 +193,13 @@ __device__ __forceinline__ int split_tokens_from(int steps, int longest, const S
 // first split pay for reading the lengths: 1 to 64 of 64 tokens under tables
 // of several pages 0.5 to 0.8 us of 6 to 9.
 // Whole steps, not whole pages.  With work items the pre-pass applies the
-// rule and leaves its result in rule.info.  Measured against the shape's split, us:
-// batch 16, 64 to 4096 tokens under 128-entry tables 77 -> 23 (the layer's
-// step), 8 x 1000 under 128 entries 53 -> 13, 1 x 512 18.6 -> 11.2, 1 x 4096
-// 19.4 -> 13.2.  Every wave of the split kernel and of the
-// merges computes the same value.  (batch <= 4096 and max_tokens <= 2^22
-// where it adapts: the sum of steps stays within an int.)
+// rule and leaves its result in rule.info.  Measured against the shape's
+// split (device time of the call, 32 q / 8 kv heads, us): 16 sequences of 64
+// to 4096 tokens under 128-entry tables 67 -> 14.5, 8 x 1000 under 128 51 ->
+// 10.6, 64 x 1000 under 128 (work items) 56 -> 32, 1 x 512 15.3 -> 8.5, 1 x
+// 4096 16.0 -> 10.8.  Every wave of the split kernel and of the merges
+// computes the same value.  (batch <= 4096 and max_tokens <= 2^22 where it
+// adapts: the sum of steps stays within an int.)
 // `own` is this lane's length, loaded early so that it shares the round trip
 // of the caller's first reads; `len` is the caller's sequence's.
 __device__ __forceinline__ int lane_length(const int32_t* __restrict__ seqlens,
@@ -959,7 +961,7 @@ __global__ __launch_bounds__(kOrderThreads) void decode_order_kernel(
 // multiple of 16 leaves the last unit's surplus lanes idle (head_ok false)
 static int qgroups_of(int group) { return (group + 15) / 16; }
 
-// Whether a decode shape runs compacted work items longest-first: split
+// Whether a decode shape runs compacted work items, the long ones first: split
 // grids of many rounds (over kWideGridMax eight-wave workgroups), where a
 // long sequence dispatched late sets the makespan and most workgroups are
 // empty splits (ragged batch 256: 423-426 against 454-457 us).  Shapes
@@ -983,7 +985,7 @@ template <typename T>
 static hipError_t launch_decode(const DecodeArgs& a, int batch, hipStream_t stream) {
   // One 8-wave workgroup (128 KB of LDS) fills a CU.  A grid of at most
   // kWideGridMax of those runs in about two rounds; a larger grid runs in
-  // many, over the longest-first work items of the pre-pass.  Beyond the
+  // many, over the work items of the pre-pass.  Beyond the
   // items' limits (and where a kv head group has fewer than eight units),
   // the last round's tail halves with 4-wave workgroups (two per CU):
   // ragged batch 256 in row order, 452 against 491 us.  The Qwen3-8B batch

@@ -696,8 +696,8 @@ static hipError_t launch_prefill(const PrefillArgs& a, int num_seqs, int64_t qbl
 // workgroups are resident per CU, 512 on the chip, and a second one costs the
 // first little (a tile takes 3.0 us unsplit, 3.2 us beside other ranges, 3.9
 // us beside another workgroup), so a grid of at most 256 is split until it
-// fills them (768 or 1024 instead: 120-134 against 106 us on 512 new over
-// 7680 cached tokens, with the store), where the shorter chain saves more
+// fills them (768 or 1024 instead: 13 and 26% slower on 512 new over 7680
+// cached tokens), where the shorter chain saves more
 // than the merge costs: its launch, 5 us, and 1 KB per row and split at 6
 // TB/s.  Unsplit against split (fp16, 32 q / 8 kv heads, new/cached, the
 // call alone, us): 512/7680 191 -> 83, 128/7680 182 -> 41, 512/1000 42.2 ->
