@@ -587,12 +587,15 @@ def test_decode_splits_follow_the_lengths_of_each_replay():
     # no full split, only full splits, ties, empty sequences; splits that
     # follow the lengths under tables of 128 entries (32 splits, 40 sequences)
     ([1 + i % 3 for i in range(40)], 128),
-    ([0] * 39 + [9000], 128), ([0] * 40, 128), ([0] * 39 + [1], 128), ([1024] * 20 + [0] * 5 + [2048, 4096] * 8, 128),
+    ([0] * 39 + [9000], 128), ([0] * 40, 128), ([0] * 39 + [1], 128),
+    ([1024] * 20 + [0] * 5 + [2048, 4096] * 8, 128),
     ([64 * (1 + i % 7) + i % 2 for i in range(40)], 128),
     # contexts short enough, and rows many enough, that none is split; one
     # that is; steps of 32 tokens at their edges
     ([33 + i % 128 for i in range(128)], 128), ([31 + i % 3 for i in range(128)], 128),
     ([64 + i % 66 for i in range(127)] + [2000], 128),
+    # more sequences than the pre-pass has threads
+    ([1 + 7 * i % 300 for i in range(299)] + [1500], 40), ([90] * 257, 8),
     # tables that fit (16 splits): the shape's own split
     ([4 * 256 * (1 + i % 16) - i % 5 for i in range(40)], 64),
 ])
